@@ -8,14 +8,9 @@
 // MFMA (v_mfma_f32_16x16x32_bf16: A = 16 vocab rows x 32 k, B = 32 k x 16
 // batch rows, C = 16 x 16 fp32).  Two stream-ordered launches:
 //
-//   1. head_tiles   grid (ceil(V / 512), ceil(B / (16 NB))), 16 waves each.
-//                   A wave owns 32 vocab rows (two 16-row MFMA tiles) and
-//                   the workgroup's 16 NB batch rows, and runs the whole k
-//                   loop: the head weights are streamed once from HBM (each
-//                   element read by one lane), the hidden states are staged
-//                   in LDS once per workgroup.  The
-//                   accumulators are reduced in registers and LDS to one
-//                   64-bit key per (workgroup, batch row): the orderable
+//   1. head_wide    one workgroup per (vocab tile, batch tile of up to 256
+//                   rows): the projection, reduced in registers and LDS to
+//                   one 64-bit key per (vocab tile, batch row): the orderable
 //                   logit above the complement of the vocab id, so the
 //                   largest key is the largest logit with the lowest id on
 //                   ties, and a NaN logit (key above +inf) the first NaN --
@@ -24,8 +19,6 @@
 //
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-#include <mutex>
 
 #include "cx_device.hpp"
 #include "cx_internal.hpp"
@@ -39,20 +32,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int HEAD_WG = 256;                 // merge workgroup
-constexpr int HEAD_NW = 16;                  // waves per tile workgroup
-constexpr int HEAD_MT = 2;                   // 16-row vocab tiles per wave
-constexpr int HEAD_VT = HEAD_NW * 16 * HEAD_MT;   // vocab rows per workgroup
-constexpr int HEAD_KB = 128;                 // k per block (4 MFMA slices)
-constexpr int HEAD_LDS = 152 * 1024;         // hidden-state chunk in LDS (at most)
+constexpr int HEAD_KB = 128;                 // D is a multiple of this
 
 struct HeadArgs {
   const uint16_t* hidden;   // [B, ldh] bf16 bits
   const uint16_t* weight;   // [V, ldw] bf16 bits
   int64_t ldh, ldw;
   int B, D, V;
-  uint64_t* part;           // [gridDim.x, B] keys
-  int nvt;                  // gridDim.x
-  int kc;                   // k per LDS chunk of hidden states
+  uint64_t* part;           // [B, nvt] keys
+  int nvt;                  // vocab tiles
   int32_t* out_id;
   float* out_max;           // nullable [B]
   float* out_logits;        // nullable [B, V] (verification)
@@ -70,114 +58,198 @@ __device__ __forceinline__ uint64_t head_key(float x, int v) {
   return ((uint64_t)k << 32) | (uint32_t)~(uint32_t)v;
 }
 
-// One k block of a wave's weights: its two vocab tiles, 4 MFMA slices each.
-struct HeadBlock {
-  u32x4 w[HEAD_MT][4];
+// A wave owns 16 MT vocab rows and all the workgroup's 16 NT batch rows, so
+// every weight element is loaded by one lane, straight into registers, and
+// the weights are read once for up to 256 batch rows; the hidden states (2 MB
+// at B = 256, D = 4096: the L2 holds them) pass through LDS in stages of 64 k.
+//
+//  * Bound: HBM (1.05 GB of weights at V = 128256, D = 4096: 146 us at the
+//    rate a large read reaches here) up to B = 256, where the MFMA time
+//    is 108 us at the dense peak.
+//  * Both operands are requested WIDE_AHEAD stages before they are used: the
+//    weights into a register ring, the hidden states by loads that write LDS
+//    directly (no registers held, and in issue order with the weights, so
+//    waiting for a stage's hidden states leaves the later stages' weights in
+//    flight; staged through registers, that wait drains the weight ring).
+//    One barrier per stage: after it every wave's share of the stage is in
+//    LDS, and every wave is done with the stage before, whose buffer the
+//    next request then overwrites.
+//  * LDS layout: a stage row is 64 k = 8 chunks of 16 bytes; chunk c of row r
+//    is at position c ^ (r & 7), so the 8 rows an operand read touches at a
+//    time fall in different banks.  The permutation is in the global address
+//    each lane loads from (a direct-to-LDS load writes lane order).
+//  * Order of k (NSEG = 4): with rows a multiple of 4096 bytes apart, every
+//    workgroup that walks k from 0 asks the same few memory channels at a
+//    time.  The workgroups therefore start at different quarters of k and
+//    wrap around.  Each quarter has its own accumulators and the four sums
+//    are added in one fixed order, so a weight row gives the same logit
+//    wherever it lies (equal rows still tie).  Measured at V = 128256,
+//    D = 4096: B = 32 213 -> 189 us, B = 64 228 -> 195 us (with rows padded
+//    by 128 bytes: 184 and 195 us); two starts instead of four give nothing,
+//    and for larger batches four sets of accumulators do not fit.
+//  * Measured, B = 256, V = 128256, D = 4096: 305 us, 880 TFLOP/s (1436 us with
+//    32 batch rows per pass over the weights); B = 128 246 us (was 757 us);
+//    B = 16, V = 32000 50 us (131 us with 512 vocab rows a workgroup, which
+//    left 193 of the 256 CUs without one).
+constexpr int WIDE_SK = 64;                  // k per stage
+constexpr int WIDE_AHEAD = 3;                // stages requested ahead
+constexpr int WIDE_RING = WIDE_AHEAD + 1;    // stage buffers
+
+template <int MT>
+struct WideStage {
+  u32x4 w[MT][2];                            // 16 rows x 32 k per operand
 };
 
-__device__ __forceinline__ void head_load(HeadBlock& x, const uint16_t* const (&wp)[HEAD_MT],
-                                          int kb) {
-#pragma unroll
-  for (int m = 0; m < HEAD_MT; ++m)
-#pragma unroll
-    for (int s = 0; s < 4; ++s) x.w[m][s] = ld16(wp[m] + kb + 32 * s);
+// s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14;
+// expcnt and lgkmcnt at their "no wait" values).
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-// The block's MFMAs; the hidden-state operands come from the LDS chunk
-// (row r of the chunk at hs + r * hstride, this lane's k offset applied).
-template <int NB>
-__device__ __forceinline__ void head_mfma(const HeadBlock& x, const CX_LDS uint16_t* hs,
-                                          int hstride, int kc, f32x4 (&acc)[HEAD_MT][NB]) {
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    u32x4 h[NB];
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-      h[n] = *(const CX_LDS u32x4*)(hs + (size_t)16 * n * hstride + kc + 32 * s);
-#pragma unroll
-    for (int m = 0; m < HEAD_MT; ++m)
-#pragma unroll
-      for (int n = 0; n < NB; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, x.w[m][s]), __builtin_bit_cast(bf16x8, h[n]), acc[m][n],
-            0, 0, 0);
-  }
-}
-
-// Workgroups of HEAD_NW waves, HEAD_NW * 32 vocab rows.  The hidden states
-// of the workgroup's 16 NB batch rows are staged in LDS a chunk of KC k at
-// a time (rows padded by 16 bytes so the 16 rows of an MFMA operand fall in
-// different banks); each wave streams its weights through a register ring
-// of DEPTH blocks, so DEPTH - 1 blocks' loads are in flight while one is
-// multiplied.
-template <int NB, int DEPTH>
-__global__ __launch_bounds__(HEAD_NW * 64) void head_tiles(HeadArgs A) {
-  extern __shared__ __align__(16) unsigned char head_lds[];
-  __shared__ uint64_t s_key[HEAD_NW][16 * NB];
-  CX_LDS uint16_t* const hsh = to_lds((uint16_t*)head_lds);
+template <int NT, int MT, int NW, int NSEG>
+__global__ __launch_bounds__(NW * 64, 1) void head_wide(HeadArgs A) {
+  constexpr int ROWS = 16 * NT;
+  constexpr int NH = 2 * NT / NW;            // direct-to-LDS loads a wave issues per stage
+  static_assert(2 * NT % NW == 0, "a stage's rows divide over the waves");
+  // one array per stage buffer: the compiler then knows that a read of one
+  // does not wait for the loads that write another
+  __shared__ __align__(16) uint16_t s_h0[ROWS * WIDE_SK];
+  __shared__ __align__(16) uint16_t s_h1[ROWS * WIDE_SK];
+  __shared__ __align__(16) uint16_t s_h2[ROWS * WIDE_SK];
+  __shared__ __align__(16) uint16_t s_h3[ROWS * WIDE_SK];
+  __shared__ uint64_t s_key[NW][ROWS];
   const int w = wave_id(), l = lane_id();
   const int g = l >> 4, c = l & 15;
-  const int v0 = blockIdx.x * (HEAD_NW * 16 * HEAD_MT) + w * 16 * HEAD_MT;
-  const int b0 = blockIdx.y * 16 * NB;
-  const int KC = A.kc;                   // k per staged chunk (a multiple of HEAD_KB)
-  const int hstride = KC + 8;            // LDS row stride, in bf16
-  // the weight rows this lane loads (clamped into the matrix; keys of rows
-  // past V are never used); slice s of lane group g is k = kb + 32 s + 8 g
-  // + i, so each load instruction reads 64 contiguous bytes of 16 rows
-  const uint16_t* wp[HEAD_MT];
+  const int nby = (A.B + ROWS - 1) / ROWS;
+  // batch tiles of one vocab tile are neighbours in the dispatch order, so
+  // they find the weights in the Infinity Cache
+  const int vt = blockIdx.x / nby;
+  const int b0 = (int)(blockIdx.x - (unsigned)vt * nby) * ROWS;
+  const int v0 = (vt * NW + w) * 16 * MT;
+  const int S = A.D / WIDE_SK;
+  const uint16_t* wp[MT];
 #pragma unroll
-  for (int m = 0; m < HEAD_MT; ++m)
+  for (int m = 0; m < MT; ++m)
     wp[m] = A.weight + (size_t)min(v0 + 16 * m + c, A.V - 1) * A.ldw + 8 * g;
-  const CX_LDS uint16_t* const hs = hsh + (size_t)c * hstride + 8 * g;
-  f32x4 acc[HEAD_MT][NB];
+  // direct-to-LDS load j of this wave: rows (j NW + w) 8 .. + 7
+  const uint16_t* hp[NH];
 #pragma unroll
-  for (int m = 0; m < HEAD_MT; ++m)
+  for (int j = 0; j < NH; ++j) {
+    const int r = (j * NW + w) * 8 + (l >> 3);
+    hp[j] = A.hidden + (size_t)min(b0 + r, A.B - 1) * A.ldh + 8 * ((l & 7) ^ (l >> 3));
+  }
+  // this workgroup's first segment; neighbours in time and on an XCD differ
+  const int phase = __builtin_amdgcn_readfirstlane((vt + (vt >> 3)) % NSEG);
+  const int rot = phase * (S / NSEG);
+  f32x4 acc[NSEG][MT][NT];
 #pragma unroll
-    for (int n = 0; n < NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  HeadBlock ring[DEPTH];
-  for (int k0 = 0; k0 < A.D; k0 += KC) {
-    const int kn = min(KC, A.D - k0);
-    // the chunk's first weight blocks, then the hidden states into LDS
+  for (int j = 0; j < NSEG; ++j)
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-      if (d * HEAD_KB < kn) head_load(ring[d], wp, k0 + d * HEAD_KB);
-    if (k0 > 0) __syncthreads();         // every wave is done with the last chunk
-    for (int i = threadIdx.x; i < 16 * NB * (kn / 8); i += HEAD_NW * 64) {
-      const int r = i / (kn / 8), e = (i % (kn / 8)) * 8;
-      const uint16_t* src = A.hidden + (size_t)min(b0 + r, A.B - 1) * A.ldh + k0 + e;
-      *(CX_LDS u32x4*)(hsh + (size_t)r * hstride + e) = *(const u32x4*)src;
-    }
-    __syncthreads();
-    for (int kb = 0; kb < kn; kb += DEPTH * HEAD_KB) {
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        const int k = kb + d * HEAD_KB;
-        if (k >= kn) break;
-        const int kx = k + (DEPTH - 1) * HEAD_KB;
-        if (kx < kn) head_load(ring[(d + DEPTH - 1) % DEPTH], wp, k0 + kx);
-        head_mfma<NB>(ring[d], hs, hstride, k, acc);
+      for (int n = 0; n < NT; ++n) acc[j][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  WideStage<MT> ring[WIDE_RING];
+
+  // Request the s-th stage in this workgroup's order (clamped to the last
+  // one, so every stage issues the same number of loads and the counted
+  // waits hold to the end).
+  auto request = [&](int s, uint16_t* buf, WideStage<MT>& x) {
+    int ks = min(s, S - 1) + rot;
+    if (NSEG > 1 && ks >= S) ks -= S;
+    const int k = ks * WIDE_SK;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(hp[j] + k),
+                                       to_lds(buf + (j * NW + w) * 8 * WIDE_SK), 16, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) x.w[m][t] = ld16(wp[m] + k + 32 * t);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // this lane's operand chunk in a stage buffer: row c of tile 0, slice 0
+  const int lofs = c * WIDE_SK + 8 * (g ^ (c & 7));
+  auto multiply = [&](const uint16_t* buf, const WideStage<MT>& x, f32x4 (&acc)[MT][NT]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const u32x4 h = *(const CX_LDS u32x4*)(to_lds((uint16_t*)buf) + (lofs ^ (32 * t)) +
+                                               n * 16 * WIDE_SK);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, x.w[m][t]), __builtin_bit_cast(bf16x8, h), acc[m][n],
+              0, 0, 0);
       }
+  };
+  // Stage s has arrived once at most the later stages' loads are outstanding.
+  auto step = [&](int s, uint16_t* cur, const WideStage<MT>& x, uint16_t* nxt, WideStage<MT>& y,
+                  f32x4 (&acc)[MT][NT]) {
+    wait_vm<(WIDE_AHEAD - 1) * (NH + 2 * MT)>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    request(s + WIDE_AHEAD, nxt, y);
+    multiply(cur, x, acc);
+    asm volatile("" ::: "memory");
+  };
+
+  request(0, s_h0, ring[0]);
+  request(1, s_h1, ring[1]);
+  request(2, s_h2, ring[2]);
+  int s = 0;
+#pragma unroll
+  for (int j = 0; j < NSEG; ++j) {
+    const int end = NSEG == 1 ? S : (j + 1) * (S / NSEG);
+    for (; s + WIDE_RING <= end; s += WIDE_RING) {
+      step(s, s_h0, ring[0], s_h3, ring[3], acc[j]);
+      step(s + 1, s_h1, ring[1], s_h0, ring[0], acc[j]);
+      step(s + 2, s_h2, ring[2], s_h1, ring[1], acc[j]);
+      step(s + 3, s_h3, ring[3], s_h2, ring[2], acc[j]);
     }
   }
-  // lane (g, c) holds logits of vocab rows v0 + 16 m + 4 g + j (j < 4) at
-  // batch row b0 + 16 n + c
+  if (NSEG == 1 && s < S) {                  // S is even
+    step(s, s_h0, ring[0], s_h3, ring[3], acc[0]);
+    step(s + 1, s_h1, ring[1], s_h0, ring[0], acc[0]);
+  }
+  wait_vm<0>();                              // the last requests write LDS: end them first
+  // the segments' sums, added in the order of k whatever order they came in
+  // (acc[j] is segment (phase + j) % NSEG)
+  if (NSEG > 1) {
 #pragma unroll
-  for (int n = 0; n < NB; ++n) {
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < NSEG; ++p)
+          if (phase == p)
+            sum = (acc[(NSEG - p) % NSEG][m][n] + acc[(NSEG - p + 1) % NSEG][m][n]) +
+                  (acc[(NSEG - p + 2) % NSEG][m][n] + acc[(NSEG - p + 3) % NSEG][m][n]);
+        acc[0][m][n] = sum;
+      }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
     const int b = b0 + 16 * n + c;
     uint64_t key = 0;
 #pragma unroll
-    for (int m = 0; m < HEAD_MT; ++m)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int v = v0 + 16 * m + 4 * g + j;
-        const float x = acc[m][n][j];
+        const float x = acc[0][m][n][j];
         if (v < A.V) {
           const uint64_t k = head_key(x, v);
           key = k > key ? k : key;
           if (A.out_logits && b < A.B) A.out_logits[(size_t)b * A.V + v] = x;
         }
       }
-    // the four lane groups of column c
     uint64_t o = __shfl_xor(key, 16);
     key = o > key ? o : key;
     o = __shfl_xor(key, 32);
@@ -185,12 +257,11 @@ __global__ __launch_bounds__(HEAD_NW * 64) void head_tiles(HeadArgs A) {
     if (g == 0) s_key[w][16 * n + c] = key;
   }
   __syncthreads();
-  const int t = threadIdx.x;
-  if (t < 16 * NB && b0 + t < A.B) {
+  for (int t = threadIdx.x; t < ROWS && b0 + t < A.B; t += NW * 64) {
     uint64_t key = s_key[0][t];
 #pragma unroll
-    for (int k = 1; k < HEAD_NW; ++k) key = s_key[k][t] > key ? s_key[k][t] : key;
-    A.part[(size_t)(b0 + t) * A.nvt + blockIdx.x] = key;
+    for (int k = 1; k < NW; ++k) key = s_key[k][t] > key ? s_key[k][t] : key;
+    A.part[(size_t)(b0 + t) * A.nvt + vt] = key;
   }
 }
 
@@ -225,34 +296,62 @@ __global__ __launch_bounds__(HEAD_WG) void head_merge(HeadArgs A) {
   }
 }
 
-// k per LDS chunk for nb batch tiles: the largest multiple of HEAD_KB whose
-// padded rows fit HEAD_LDS, at most D.
-static int head_kc(int D, int nb) {
-  int kc = (HEAD_LDS / (16 * nb * 2) - 8) / HEAD_KB * HEAD_KB;
-  return kc < D ? kc : D;
+// The launch of a batch of B rows over V vocab rows: batch tiles of 32, 64,
+// 128 or 256 rows, and workgroups of 64 (4 waves), 128 or 256 vocab rows (8
+// waves of 16 or 32).
+struct HeadPlan {
+  int nt;            // index of the batch tile: 32 << nt rows
+  int vt;            // vocab rows per workgroup
+  int nby;           // batch tiles
+};
+static HeadPlan head_plan(int B, int V) {
+  HeadPlan p;
+  p.nt = B <= 32 ? 0 : B <= 64 ? 1 : B <= 128 ? 2 : 3;
+  p.nby = (B + (32 << p.nt) - 1) / (32 << p.nt);
+  if (p.nt == 0) {
+    // small workgroups balance best at every V: 120 against 134 us for 128
+    // vocab rows at V = 80000, 11 against 15 us at V = 4080
+    p.vt = 64;
+  } else if (p.nt < 3) {
+    // 128 vocab rows (B = 64: 57 against 62 us at V = 32000) once they fill
+    // most of the CUs; below, 64 (18 against 24 us at V = 16000)
+    p.vt = V > 128 * 160 ? 128 : 64;
+  } else {
+    // one workgroup per CU at a time: the fewest rounds over the 256 CUs,
+    // each weighted by its measured time in us (D = 4096)
+    const int vts[3] = {256, 128, 64}, us[3] = {150, 92, 67};
+    long best = 0;
+    for (int i = 0; i < 3; ++i) {
+      const long wg = (long)((V + vts[i] - 1) / vts[i]) * p.nby;
+      const long cost = (wg + 255) / 256 * us[i];
+      if (i == 0 || cost < best) { best = cost; p.vt = vts[i]; }
+    }
+  }
+  return p;
 }
 
 int launch_head(const HeadArgs& A0, hipStream_t s) {
   HeadArgs A = A0;
-  // 16-row batch tiles per wave (four spill: their accumulators and a ring
-  // of two blocks exceed the 128 VGPRs of a 16-wave workgroup)
-  const int nb = A.B >= 32 ? 2 : 1;
-  A.kc = head_kc(A.D, nb);
-  const dim3 grid(A.nvt, (A.B + 16 * nb - 1) / (16 * nb));
-  const uint32_t lds = (uint32_t)(16 * nb * (A.kc + 8) * 2);
-  const dim3 blk(HEAD_NW * 64);
+  const HeadPlan p = head_plan(A.B, A.V);
+  A.nvt = (A.V + p.vt - 1) / p.vt;
+  // weight rows a multiple of 4096 bytes apart: four starting points in k
+  // (each quarter a whole number of ring turns)
+  const bool seg = A.ldw % 2048 == 0 && A.D % (4 * WIDE_RING * WIDE_SK) == 0;
   using K = void (*)(HeadArgs);
-  static const K kern[2] = {head_tiles<1, 3>, head_tiles<2, 2>};
-  const int v = nb - 1;
-  // the dynamic-LDS limit raised once per variant to the most any launch takes
-  static std::once_flag once[2];
-  hipError_t err = hipSuccess;
-  std::call_once(once[v], [&] {
-    err = hipFuncSetAttribute((const void*)kern[v], hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HEAD_LDS);
-  });
-  if (err != hipSuccess) return (int)err;
-  timed_launch(CX_KERNEL_LMHEAD, kern[v], grid, blk, lds, s, A);
+  K k;
+  switch (p.nt) {
+    case 0: k = seg ? head_wide<2, 1, 4, 4> : head_wide<2, 1, 4, 1>; break;
+    case 1:
+      k = p.vt == 64 ? (seg ? head_wide<4, 1, 4, 4> : head_wide<4, 1, 4, 1>)
+                     : (seg ? head_wide<4, 1, 8, 4> : head_wide<4, 1, 8, 1>);
+      break;
+    case 2: k = p.vt == 64 ? head_wide<8, 1, 4, 1> : head_wide<8, 1, 8, 1>; break;
+    default:
+      k = p.vt == 64 ? head_wide<16, 1, 4, 1>
+                     : p.vt == 128 ? head_wide<16, 1, 8, 1> : head_wide<16, 2, 8, 1>;
+  }
+  timed_launch(CX_KERNEL_LMHEAD, k, dim3((unsigned)(A.nvt * p.nby)), dim3(p.vt == 64 ? 256 : 512),
+               0, s, A);
   timed_launch(CX_KERNEL_LMHEAD_MERGE, head_merge, dim3(A.B), dim3(HEAD_WG), 0, s, A);
   return (int)hipGetLastError();
 }
@@ -263,7 +362,8 @@ extern "C" {
 
 size_t cx_lmhead_workspace_bytes(int32_t B, int32_t V) {
   if (B <= 0 || V <= 0) return 256;
-  return ((size_t)B * ((V + cx::HEAD_VT - 1) / cx::HEAD_VT) * 8 + 255) & ~(size_t)255;
+  const int vt = cx::head_plan(B, V).vt;
+  return ((size_t)B * ((V + vt - 1) / vt) * 8 + 255) & ~(size_t)255;
 }
 
 int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* weight,
@@ -285,7 +385,6 @@ int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* w
   cx::HeadArgs A;
   A.hidden = hidden; A.weight = weight; A.ldh = ldh; A.ldw = ldw;
   A.B = B; A.D = D; A.V = V;
-  A.nvt = (V + cx::HEAD_VT - 1) / cx::HEAD_VT;
   A.part = (uint64_t*)workspace;
   A.out_id = out_id; A.out_max = out_max; A.out_logits = out_logits;
   const int e = cx::launch_head(A, (hipStream_t)stream);

@@ -67,6 +67,29 @@ def test_small_shapes_logits_and_ids(B, D, V):
     _check(h, w, ids, mx, lg)
 
 
+@pytest.mark.parametrize("B,D,V", [
+    (1, 128, 63), (32, 1024, 65), (17, 2048, 641),         # 32 batch rows; k from 4 starts
+    (34, 384, 64), (64, 1024, 20481), (65, 640, 20480), (128, 128, 20545),
+    (129, 256, 16384), (200, 128, 16385), (256, 384, 40001), (257, 1024, 129)])
+def test_tile_edges(B, D, V):
+    """Every batch tile (32, 64, 128, 256 rows, two of them) and vocab tile
+    (64, 128, 256), with ragged last tiles, the shortest k and k in quarters."""
+    print(f"[gpu] lm head tile edges B={B} D={D} V={V}", flush=True)
+    rng = np.random.default_rng(B * 5 + D + V)
+    h = f32_to_bf16_bits(rng.normal(0, 1, (B, D)).astype(np.float32))
+    w = f32_to_bf16_bits(rng.normal(0, 0.05, (V, D)).astype(np.float32))
+    # copies of row 0's best weight row in other tiles, which start k elsewhere
+    src = int(H.greedy_ids(H.head_logits(h[:1], w))[0])
+    for dst in (src % 64, 64 + src % 61, V // 2, V - 1):
+        if dst < V:
+            w[dst] = w[src]
+    ids, mx, lg = _run(h, w)
+    _check(h, w, ids, mx, lg)
+    same = [v for v in range(V) if (w[v] == w[src]).all()] if V < 1000 else \
+        np.flatnonzero((w == w[src]).all(axis=1)).tolist()
+    assert len(set(lg[0, same].tolist())) == 1 and ids[0] == same[0]
+
+
 def test_ties_and_nan():
     print("[gpu] lm head ties and NaN", flush=True)
     rng = np.random.default_rng(9)
