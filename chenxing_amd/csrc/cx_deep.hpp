@@ -82,14 +82,14 @@ typedef uint32_t deep_u32x4 __attribute__((vector_size(16)));
 // The row as the passes read it.  nv values per thread per step (8 fp32 or
 // 16 bf16, 32 bytes), a step covering nv * WG ids.
 struct DeepRow {
-  __amdgpu_buffer_rsrc_t rs;  // the row, rounded up to 16 bytes (aligned rows)
+  __amdgpu_buffer_rsrc_t rs;  // the row, rounded up to 4 bytes (rows of whole dwords)
   const void* p;
   int V, nv, step;
   bool bf16;
 };
 
-// The 32 bytes holding values [e0, e0 + nv) (e0 a multiple of nv).  Aligned
-// rows: two range-checked 16-byte loads (zeros past the row, no branch), so
+// The 32 bytes holding values [e0, e0 + nv) (e0 a multiple of nv).  Rows of
+// whole dwords: two range-checked 16-byte loads (zeros past the row, no branch), so
 // the compiler can keep them in flight; other rows: value by value, zero
 // past V.
 template <bool VEC>
@@ -246,9 +246,198 @@ __device__ inline bool deep_eligible(const SampleArgs& A, int row, const cx_row_
   return m > -__builtin_inf() && m < __builtin_inf();
 }
 
-template <bool VEC>
+// ---------------------------------------------------------------- whole rows
+// Rows with no top-k, top-p or min-p and no penalty window: the draw (or,
+// with typical-p, the order's entropy) takes every element, so no candidate
+// region helps.  The fused kernel reads such a row once (whole_slice) and
+// keeps, per 1024-element chunk, the chunk's maximum and its fp64 sums
+// against it; slow_kernel's workgroup of the row then has the normaliser and
+// every chunk's place in the cumulative sum from one scan of at most ~1040
+// records, and the draw reads a single chunk (whole_finish).
+//
+// Bound: the fused kernel's slices are fp64-VALU work (one table exp per
+// element, ~25 instructions; HBM would allow 5 us for 64 rows of 128256
+// fp32) on all CUs; the finish is a chain of barriers on one CU per row.
+// Before, the row was streamed for a region it then outgrew and summed,
+// bucketed and drawn by one workgroup: 64 rows of 128256 fp32, no filter,
+// 108 us a call; typical-p 0.95 on the multi-pass path, 1225 us.
+struct WholePart {
+  double s;          // sum of exp((x - m) / T) over the chunk (NaN: a NaN or +inf element)
+  double sd;         // sum of exp((x - m) / T) (x - m) / T
+  float m;           // the chunk's maximum
+  int32_t pad;
+};
+constexpr int WCH = 1024;                     // elements per chunk
+static_assert((SLICE_MAX / WCH + 2) * sizeof(WholePart) <= CAPS * sizeof(Cand),
+              "a slice's records fit its region");
+
+// (a row without a penalty window; ln V / T > 740: P**(1/T) may underflow)
+__device__ __forceinline__ bool whole_row(const SampleArgs& A, const cx_row_params& P) {
+  return !(P.top_k > 0 && P.top_k < A.V) && !(P.top_p < 1.0) && !(P.min_p > 0.0) &&
+         P.temperature > 0.0 && !A.out_probs && A.logV * (1.0 / P.temperature) <= 740.0;
+}
+
+// A slice's chunks: nvc of whole vectors from lo, then nsc over the rest
+// [s0, hi) (everything, on unaligned rows), 1024 ids each but the last of
+// either kind.
+struct WholeSlice {
+  int lo, s0, hi, nvc, nsc;
+  __device__ int first(int i) const { return i < nvc ? lo + i * WCH : s0 + (i - nvc) * WCH; }
+  __device__ int end(int i) const { return min(first(i) + WCH, i < nvc ? s0 : hi); }
+};
+__device__ __forceinline__ WholeSlice whole_slice_of(const SampleArgs& A, int split) {
+  WholeSlice w;
+  const int ne = A.bf16 ? 8 : 4;
+  w.lo = split * A.split_len;
+  w.hi = min(A.V, w.lo + A.split_len);
+  w.s0 = A.vec_ok && w.hi > w.lo ? w.lo + (w.hi - w.lo) / ne * ne : w.lo;
+  w.nvc = (w.s0 - w.lo + WCH - 1) / WCH;
+  w.nsc = w.hi > w.s0 ? (w.hi - w.s0 + WCH - 1) / WCH : 0;
+  return w;
+}
+
+// One chunk's record, by one wave: 16 values per lane, -inf where absent.
+__device__ __forceinline__ void whole_chunk(const float (&x)[16], double invT, const double* tab,
+                                            WholePart* out) {
+  float m = x[0];
+  bool bad = false;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    m = fmaxf(m, x[j]);
+    bad = bad || !(x[j] < __builtin_inff());
+  }
+  m = wave_reduce(m, OpMax());
+  double s = 0.0, sd = 0.0;
+  if (m > -__builtin_inff()) {
+    double sa[4] = {0.0, 0.0, 0.0, 0.0}, da[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      // (-inf: the exponential's clamp, so 0 * inf never arises)
+      const double d = fmax(((double)x[j] - (double)m) * invT, -745.2);
+      const double e = exp64_neg(d, tab);
+      sa[j & 3] += e;
+      da[j & 3] += e * d;
+    }
+    s = wave_reduce((sa[0] + sa[1]) + (sa[2] + sa[3]), OpAdd());
+    sd = wave_reduce((da[0] + da[1]) + (da[2] + da[3]), OpAdd());
+  }
+  if (ballot(bad)) s = __builtin_nan("");
+  if (lane_id() == 0) {
+    out->s = s;
+    out->sd = sd;
+    out->m = m;
+  }
+}
+
+// Outcomes of whole_finish.
+constexpr int WHOLE_OPEN = 0;      // degenerate or too near a step: the exact path
+constexpr int WHOLE_DONE = 1;      // drawn
+constexpr int WHOLE_TYP = 2;       // typical-p row: Z holds its sums for deep_row
+struct WholeSums {
+  double M;          // row maximum
+  double c;          // -sum P d, d = (x - M) / T: the entropy less log S
+  double wt;         // 1 / sum exp(d)
+};
+
+// All threads of the workgroup; every thread gets the same result.  The
+// typical order's distance |log P + H| (sampler.py:97-98) is |d + c|.
+__device__ inline int whole_finish(const SampleArgs& A, int row, const cx_row_params& P,
+                                   double* red_d, int* red_i, WholeSums& Z) {
+  __shared__ double tab[64];
+  __shared__ double s_w[2 * NWAVE + 4];
+  __shared__ double s_off;
+  __shared__ int s_ok;
+  const int t = threadIdx.x;
+  const double invT = 1.0 / P.temperature;
+  load_exp64_tab(tab);
+  // records 2t and 2t + 1, slice by slice (V < 2^20: at most 1040 in all)
+  double ps[2] = {0.0, 0.0}, pd[2] = {0.0, 0.0};
+  float pm[2] = {-__builtin_inff(), -__builtin_inff()};
+  {
+    int base = 0;
+    for (int sl = 0; sl < A.nsplit; ++sl) {
+      const WholeSlice W = whole_slice_of(A, sl);
+      const int n = W.nvc + W.nsc;
+      const WholePart* q = (const WholePart*)(A.cands + ((size_t)row * A.nsplit + sl) * CAPS);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int i = 2 * t + j - base;
+        if (i >= 0 && i < n) { ps[j] = q[i].s; pd[j] = q[i].sd; pm[j] = q[i].m; }
+      }
+      base += n;
+    }
+  }
+  const float Mf = block_max(fmaxf(pm[0], pm[1]), (float*)red_i, -__builtin_inff());
+  const double M = (double)Mf;
+  double dsum = 0.0;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (pm[j] > -__builtin_inff()) {
+      const double dm = ((double)pm[j] - M) * invT;
+      const double f = exp64_neg(dm, tab);
+      dsum += f * (pd[j] + ps[j] * dm);
+      ps[j] *= f;
+    }
+  }
+  const double S = block_sum(ps[0] + ps[1], red_d);
+  if (!(Mf > -__builtin_inff() && Mf < __builtin_inff() && S > 0.0 && S < __builtin_inf()))
+    return WHOLE_OPEN;
+  if (P.typical_p < 1.0) {
+    Z.M = M;
+    Z.c = -block_sum(dsum, red_d) / S;
+    Z.wt = 1.0 / S;
+    return Z.c >= 0.0 ? WHOLE_TYP : WHOLE_OPEN;
+  }
+  // the chunk holding u * S (sampler.py:126-127), then the element in it
+  const double t2 = A.u[row] * S, tolS = DTOL * S;
+  const double before = block_excl_scan_d(ps[0] + ps[1], s_w);
+  const int mine = before + ps[0] > t2 ? 2 * t
+                   : before + ps[0] + ps[1] > t2 ? 2 * t + 1 : INT_MAX;
+  const int ci = block_min(mine, red_i, INT_MAX);
+  if (ci == INT_MAX) return WHOLE_OPEN;
+  if (mine == ci) s_off = (ci & 1) ? before + ps[0] : before;
+  int lo = 0, hi = 0;
+  {
+    int base = 0;
+    for (int sl = 0; sl < A.nsplit; ++sl) {
+      const WholeSlice W = whole_slice_of(A, sl);
+      const int n = W.nvc + W.nsc;
+      if (ci >= base && ci < base + n) { lo = W.first(ci - base); hi = W.end(ci - base); }
+      base += n;
+    }
+  }
+  double e = 0.0;
+  if (lo + t < hi) {
+    const char* rowp = (const char*)A.logits + (size_t)row * (size_t)A.ld * (A.bf16 ? 2 : 4);
+    const float x = A.bf16 ? __uint_as_float((uint32_t)((const uint16_t*)rowp)[lo + t] << 16)
+                           : ((const float*)rowp)[lo + t];
+    e = exp64_neg(((double)x - M) * invT, tab);
+  }
+  const double r = block_excl_scan_d(e, s_w) + s_off;      // (its barriers publish s_off)
+  const int hit = block_min(r + e > t2 ? t : INT_MAX, red_i, INT_MAX);
+  if (hit == INT_MAX) return WHOLE_OPEN;
+  if (t == hit) s_ok = r + e > t2 + tolS && r < t2 - tolS ? 1 : 0;
+  __syncthreads();
+  if (!s_ok) return WHOLE_OPEN;
+  if (t == 0) {
+    A.out_id[row] = lo + hit;
+    A.row_status[row] = CX_ROW_OK;
+  }
+  return WHOLE_DONE;
+}
+
+// TYP: a typical-p row with no other filter (sampler.py:95-105).  The same
+// passes in the typical order, ascending |d + c| with d = (x - M) / T and
+// c = -sum P d (whole_finish): the buckets are linear in that distance (in
+// fp64, so the two sides of the order compare exactly), the terms are the
+// probabilities e wt themselves, and a bucket sums them in units of 2^-60 (at
+// most 1 in all, so one scale serves every bucket).  A cut beside an element
+// of the other side whose distance differs by less than 1e-11 is left to
+// the multi-pass path.
+template <bool VEC, bool TYP>
 __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, const cx_row_params& P,
-                                     double M, unsigned char* dyn, double* red_d, int* red_i) {
+                                     double M, unsigned char* dyn, double* red_d, int* red_i,
+                                     double c, double wt) {
   __shared__ double tab[64];
   __shared__ double s_d[2 * NWAVE + 4];
   __shared__ double s_wm[NWAVE];                     // kept mass per wave range / sixteenth
@@ -283,6 +472,20 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   // step, so each workgroup step lies in one range
   const int L = ((V + NWAVE * R.step - 1) / (NWAVE * R.step)) * R.step;
   const int nsteps = (V + R.step - 1) / R.step;
+  // the typical order's distance of value x, its bucket (-1 past the span),
+  // and the fixed-point scale of a bucket's terms
+  auto dist = [&](float x) { return fabs(((double)x - M) * invT + c); };
+  auto bucket = [&](float x) -> int {
+    if constexpr (!TYP) return deep_bucket(x, Mf, invTf);
+    const double v = dist(x) * (double)DSCALE;
+    return v < (double)DNB ? (int)v : -1;
+  };
+  auto scale = [&](int b) { return deep_pow2(TYP ? 60 : deep_scale(b)); };
+  auto unscale = [&](int b) { return deep_pow2(TYP ? -60 : -deep_scale(b)); };
+  auto term = [&](float x) { return TYP ? deep_term(x, M, invT, tab) * wt : deep_term(x, M, invT, tab); };
+  auto term16 = [&](uint32_t code) {
+    return TYP ? deep_term16(code, ta, tb, tc) * wt : deep_term16(code, ta, tb, tc);
+  };
   for (int b = t; b < DNB; b += WG) h[b] = 0ull;
   if (t < 2 * NWAVE) s_corr[t] = 0ull;
   if (t == 0) s_i[0] = 0;
@@ -302,12 +505,11 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       if (j >= nv || e0 + j >= V) break;
       const float x = deep_val(R, wd, j);
       if (!(x == x) || x > Mf) { bad = 1; continue; }
-      const int b = deep_bucket(x, Mf, invTf);
+      const int b = bucket(x);
       // (the tables leave out terms below the span: at most V exp(-40) in all)
-      const double ev = !use_tab ? deep_term(x, M, invT, tab)
-                                 : (b >= 0 ? deep_term16(deep_code(wd, j), ta, tb, tc) : 0.0);
+      const double ev = !use_tab ? term(x) : (b >= 0 ? term16(deep_code(wd, j)) : 0.0);
       s += ev;
-      if (b >= 0) atomicAdd(h + b, (unsigned long long)(ev * deep_pow2(deep_scale(b))));
+      if (b >= 0) atomicAdd(h + b, (unsigned long long)(ev * scale(b)));
     }
     const int r = (k * R.step) / L;
     if ((k + 1) * R.step % L == 0 || k + 1 == nsteps) {
@@ -315,7 +517,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       __syncthreads();
       double v = 0.0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v += (double)h[4 * t + j] * deep_pow2(-deep_scale(4 * t + j));
+      for (int j = 0; j < 4; ++j) v += (double)h[4 * t + j] * unscale(4 * t + j);
       v = row_reduce(v, OpAdd());
       for (int rr = r; rr < (k + 1 == nsteps ? NWAVE : r + 1); ++rr)
         if ((t & 15) == 0) C[rr * DNCB + (t >> 4)] = v;
@@ -327,17 +529,18 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   const double tolS = DTOL * S;
 
   // ---- the cut: first non-empty bucket whose inclusive sum reaches top_p * S
-  const bool cut = P.top_p < 1.0;
+  const bool cut = TYP || P.top_p < 1.0;
   float xcut = -__builtin_inff();
+  double dcut = 0.0;                                 // TYP: the cut distance
   int g0 = 0, gn = 0, gj = 0;                        // the cut value's group: none
   int bs = DNB;                                      // no cut: every bucket above it
   if (cut) {
-    const double tgt = P.top_p * S;
+    const double tgt = (TYP ? P.typical_p : P.top_p) * S;
     double vb[4];
     double c4 = 0.0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      vb[j] = (double)h[4 * t + j] * deep_pow2(-deep_scale(4 * t + j));
+      vb[j] = (double)h[4 * t + j] * unscale(4 * t + j);
       c4 += vb[j];
     }
     double before = block_excl_scan_d(c4, s_d);
@@ -363,7 +566,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     // coarse bucket above it (the copies end at coarse-bucket boundaries)
     const bool corr = P.min_p <= 0.0;
     const int cb0 = (bs / DCB) * DCB;
-    const double fc = deep_pow2(deep_scale(cb0));
+    const double fc = scale(cb0);
     unsigned long long acc = 0ull;
     deep_stream<VEC>(R, 0, R.step, t, nsteps, [&](int k, const uint32_t (&wd)[DW]) {
       const int e0 = k * R.step + nv * t;
@@ -371,7 +574,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       for (int j = 0; j < DNV; ++j) {
         if (j >= nv) break;
         const float x = deep_val(R, wd, j);
-        const int b = e0 + j < V ? deep_bucket(x, Mf, invTf) : -1;
+        const int b = e0 + j < V ? bucket(x) : -1;
         // the cut bucket's elements, placed by one LDS atomic per wave
         const bool g = b == bs;
         const uint64_t m = ballot(g);
@@ -381,14 +584,13 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
           base = __builtin_amdgcn_readfirstlane(base);
           const int pos = base + lanes_below(m);
           if (g && pos < cap) {
-            gk[pos] = d2key((double)x);
+            gk[pos] = d2key(TYP ? -dist(x) : (double)x);
             gi[pos] = e0 + j;
-            ga[pos] = 0;
+            ga[pos] = (int32_t)__float_as_uint(x);
           }
         }
         if (corr && b >= cb0 && b < bs)
-          acc += (unsigned long long)((use_tab ? deep_term16(deep_code(wd, j), ta, tb, tc)
-                                               : deep_term(x, M, invT, tab)) * fc);
+          acc += (unsigned long long)((use_tab ? term16(deep_code(wd, j)) : term(x)) * fc);
       }
       if (corr && ((k + 1) * R.step % L == 0 || k + 1 == nsteps)) {
         const unsigned long long m = wave_sum(acc);
@@ -400,14 +602,14 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     const int ng = s_i[0];
     __syncthreads();
     if (ng > cap) return false;
-    block_sort<4>(gk, gi, ga, ng);                   // value descending, id ascending
+    block_sort<4>(gk, gi, ga, ng);                   // key descending, id ascending
     // thread t: sorted entries 4t .. 4t+3, their terms and running sums
     double qv[4];
     double s4 = 0.0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e = 4 * t + j;
-      qv[j] = e < ng ? exp64_neg((key2d(gk[e]) - M) * invT, tab) : 0.0;
+      qv[j] = e < ng ? term(__uint_as_float((uint32_t)ga[e])) : 0.0;
       s4 += qv[j];
     }
     double run = above + block_excl_scan_d(s4, s_d);
@@ -429,7 +631,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     if (jstar == js) {
       // robust: this element's running sum clearly reaches the target and
       // the one before clearly does not (the first element is always kept)
-      const bool first = bs == 0 && js == 0;
+      const bool first = !TYP && bs == 0 && js == 0;
       const bool ok = cstar >= tgt + tolS && (first || cprev < tgt - tolS);
       s_i[1] = ok ? 1 : 0;
       s_g[0] = js;
@@ -445,17 +647,32 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       for (int j = 0; j < 4; ++j) {
         const int e = 4 * t + j;
         if (e < ng && gk[e] == kj) { atomicMin(&s_g[0], e); atomicMax(&s_g[1], e + 1); }
+        // (the order's other side at the very same distance)
+        if (TYP && e < ng && gk[e] == kj && ga[e] != ga[js]) s_i[1] = 0;
       }
     }
     __syncthreads();
-    xcut = (float)red_d[2 * NWAVE + 2];
+    if constexpr (TYP) {
+      if (t == 0) {
+        const double kd = key2d(gk[js]);
+        const double fr = -kd * (double)DSCALE;
+        const bool near = (s_g[0] > 0 && key2d(gk[s_g[0] - 1]) - kd < 1e-11) ||
+                          (s_g[1] < ng && kd - key2d(gk[s_g[1]]) < 1e-11) ||
+                          fabs(fr - __builtin_rint(fr)) < 1e-8;   // beside the next bucket
+        if (near) s_i[1] = 0;
+      }
+      __syncthreads();
+      if (!s_i[1]) return false;
+    }
+    if constexpr (TYP) dcut = -red_d[2 * NWAVE + 2];
+    else xcut = (float)red_d[2 * NWAVE + 2];
     g0 = s_g[0];
     gn = s_g[1] - g0;
     gj = js + 1 - g0;
     // the kept part of the cut bucket, per range: the entries above the cut
     // value and the group's survivors
     if (corr) {
-      const double fb = deep_pow2(deep_scale(bs));
+      const double fb = scale(bs);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int e = 4 * t + j;
@@ -481,10 +698,15 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     }
     return spread_keeps(lo - g0, gj, gn, V <= TIE_NET);
   };
-  auto kept_e = [&](float x, int id, int& amb) -> double {
-    const uint32_t kx = f2key(x);
-    if (!(kx > kcut || (kx == kcut && in_group(id)))) return 0.0;
-    const double ev = deep_term(x, M, invT, tab);
+  auto kept_e = [&](float x, int id, int& amb) __attribute__((always_inline)) -> double {
+    if constexpr (TYP) {
+      const double v = dist(x);
+      if (!(v < dcut || (v == dcut && in_group(id)))) return 0.0;
+    } else {
+      const uint32_t kx = f2key(x);
+      if (!(kx > kcut || (kx == kcut && in_group(id)))) return 0.0;
+    }
+    const double ev = term(x);
     if (minp > 0.0) {
       if (fabs(ev - minp) <= minp_tol) amb = 1;
       if (ev < minp) return 0.0;
@@ -494,7 +716,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   int amb = 0;
   // kept mass of ids [lo, hi) by one wave (hi - lo a multiple of 64 nv), in
   // a fixed order
-  auto wave_mass = [&](int lo, int hi) -> double {
+  auto wave_mass = [&](int lo, int hi) __attribute__((always_inline)) -> double {
     double m = 0.0;
     const int n = hi > lo ? (hi - lo) / (64 * nv) : 0;
     deep_stream<VEC>(R, lo, 64 * nv, l, n, [&](int k, const uint32_t (&wd)[DW]) {
@@ -516,8 +738,8 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       for (int cb = 0; cb < cbs; ++cb)
         m += C[t * DNCB + cb] - (t > 0 ? C[(t - 1) * DNCB + cb] : 0.0);
       if (cut)
-        m += (double)s_corr[t] * deep_pow2(-deep_scale((bs / DCB) * DCB)) +
-             (double)s_corr[NWAVE + t] * deep_pow2(-deep_scale(bs));
+        m += (double)s_corr[t] * unscale((bs / DCB) * DCB) +
+             (double)s_corr[NWAVE + t] * unscale(bs);
       s_wm[t] = m;
     }
     __syncthreads();
@@ -666,14 +888,16 @@ __device__ inline double deep_exact_sum(const SampleArgs& A, int row, double M, 
 // Samples the row and returns true, or returns false with nothing written
 // (the caller runs the multi-pass path).  All threads of the workgroup call
 // it and get the same result.  dyn: DEEP_LDS bytes; red_d, red_i: >= 2 *
-// NWAVE + 4 slots.
+// NWAVE + 4 slots.  Z: a typical-p row's sums (whole_finish), else null.
 __device__ __forceinline__ bool deep_row(const SampleArgs& A, int row, unsigned char* dyn, double* red_d,
-                                int* red_i) {
+                                int* red_i, const WholeSums* Z = nullptr) {
   const cx_row_params P = A.prm[row];
+  if (Z)             // (unaligned rows: the multi-pass path)
+    return A.vec_ok && deep_row_impl<true, true>(A, row, P, Z->M, dyn, red_d, red_i, Z->c, Z->wt);
   double M = 0.0;
   if (!deep_eligible(A, row, P, M)) return false;
-  return A.vec_ok ? deep_row_impl<true>(A, row, P, M, dyn, red_d, red_i)
-                  : deep_row_impl<false>(A, row, P, M, dyn, red_d, red_i);
+  return A.vec_ok ? deep_row_impl<true, false>(A, row, P, M, dyn, red_d, red_i, 0.0, 1.0)
+                  : deep_row_impl<false, false>(A, row, P, M, dyn, red_d, red_i, 0.0, 1.0);
 }
 
 }  // namespace cx

@@ -237,6 +237,7 @@ __device__ inline void prefix_cut(int E, const int32_t* sidx, BucketOf bucket_of
 // Outcomes of finish_row_fast.
 constexpr int FIN_PENDING = 0;   // the exact multi-pass path must take the row
 constexpr int FIN_DONE = 1;      // decided and written
+constexpr int FIN_WHOLE = 3;     // no region: a row drawn from whole (cx_deep.hpp)
 constexpr int FIN_REFINE = 2;    // region complete, but a top-p cut lies within the
                                  // normaliser's error bound: decide again with an
                                  // exact fp64 normaliser
@@ -426,6 +427,7 @@ __device__ inline int finish_row_fast(const SampleArgs& A, int row, const cx_row
   const SplitStats& me = st[lin ? ls : 0];
   const int flags = row0_reduce(lin ? me.flags : 0, OpOr());
 
+  if (flags & SF_WHOLE) return FIN_WHOLE;
   if (flags & SF_UNSUPPORTED) {
     write_row_result(A, row, CX_ROW_UNSUPPORTED, -1);
     return FIN_DONE;

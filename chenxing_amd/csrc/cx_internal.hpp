@@ -21,6 +21,8 @@ constexpr double TOL_MAX = 1e-4;          // rows whose bound exceeds this are r
 constexpr int SF_OVERFLOW = 1;            // a wave buffer flooded with ties
 constexpr int SF_UNSUPPORTED = 2;         // window longer than WIN_MAX
 constexpr int SF_INEXACT = 4;             // the slice's normaliser has no usable error bound
+constexpr int SF_WHOLE = 16;              // the row is drawn from whole: its chunks' records are in
+                                          // the slice's region area (whole_slice)
 constexpr int SF_EXACT = 8;               // sx holds the slice's fp64 normaliser (bound sxtol)
 
 
@@ -34,6 +36,9 @@ constexpr int SF_EXACT = 8;               // sx holds the slice's fp64 normalise
 constexpr int ROW_PENDING = 0x40000000;
 constexpr int ROW_REFINE = 0x40000001;
 constexpr int ROW_FINISH = 0x40000002;
+// A row drawn from whole, also in its hand-off mark: slow_kernel finishes it
+// (a sliced row's workgroup finds SF_WHOLE in the slice records).
+constexpr int ROW_WHOLE = 0x40000003;
 // In a single-slice row's hand-off mark (SampleArgs::counters), beside its
 // ROW_* value: the row may take the counted deep-nucleus path
 // (deep_candidate, top-k allowed), and it has a top-k bound.
@@ -97,7 +102,8 @@ struct SampleArgs {
   int64_t ldo;
   int32_t slow_nbw;       // multi-pass kernel: full-row bitmap words (power of two)
   int32_t slow_off_hkey, slow_off_work, slow_off_tsum, slow_lds_bytes;
-  // slow_kernel takes only rows marked ROW_PENDING (after finish16_kernel)
+  // slow_kernel takes only rows marked ROW_PENDING or ROW_WHOLE (after
+  // finish16_kernel)
   int32_t pending_only;
 };
 

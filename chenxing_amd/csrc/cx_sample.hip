@@ -760,6 +760,51 @@ __device__ __forceinline__ void stream_scalar(const char* rowp, int s0, int lo, 
   }
 }
 
+// ------------------------------------------------------------ whole rows
+// The slice's chunk records (whole_chunk, cx_deep.hpp), chunk by chunk
+// round-robin over the waves, two chunks in flight (q, qn: this wave's first
+// two, loaded by the caller).
+template <bool BF16>
+__device__ __forceinline__ void whole_slice(const WholeSlice& W, __amdgpu_buffer_rsrc_t rs,
+                                            typename Elem<BF16>::V (&q)[Elem<BF16>::U],
+                                            typename Elem<BF16>::V (&qn)[Elem<BF16>::U], int nv,
+                                            const char* rowp, double invT, const double* etab,
+                                            WholePart* parts) {
+  using E = Elem<BF16>;
+  constexpr int NE = E::NE;
+  constexpr int U = E::U;
+  static_assert(U * NE == 16 && 64 * U * NE == WCH, "chunk shape");
+  int ch = __builtin_amdgcn_readfirstlane(wave_id());
+  auto step = [&](typename E::V (&b)[U]) {
+    float x[16];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float v[NE];
+      E::unpack(b[u], v);
+      const bool in = ch * (64 * U) + u * 64 + lane_id() < nv;
+#pragma unroll
+      for (int j = 0; j < NE; ++j) x[u * NE + j] = in ? v[j] : -__builtin_inff();
+    }
+    load_chunk<BF16>(rs, min(ch + 2 * NWAVE, W.nvc), b);   // past the slice: zeros, never used
+    whole_chunk(x, invT, etab, parts + ch);
+    ch += NWAVE;
+  };
+  while (ch < W.nvc) {
+    step(q);
+    if (ch >= W.nvc) break;
+    step(qn);
+  }
+  // the elements after the last whole vector, or all of an unaligned row
+  for (int k = __builtin_amdgcn_readfirstlane(wave_id()); k < W.nsc; k += NWAVE) {
+    const int lo = W.s0 + k * WCH + lane_id();
+    float x[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      x[j] = lo + 64 * j < W.hi ? E::scalar(rowp, lo + 64 * j) : -__builtin_inff();
+    whole_chunk(x, invT, etab, parts + W.nvc + k);
+  }
+}
+
 // ------------------------------------------------------------ greedy stream
 struct GreedyState {
   float bv;
@@ -1103,7 +1148,7 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
 
   __shared__ int s_nd;
   __shared__ int s_gctr;
-  __shared__ double s_etab[EXACT ? 64 : 1];   // EXP64_TAB, for the exact sums
+  __shared__ double s_etab[64];               // EXP64_TAB, for the exact sums and whole rows
   __shared__ double w_xs[EXACT ? NWAVE : 1], w_xm[EXACT ? NWAVE : 1];
   const int row = blockIdx.x / A.nsplit;
   const int split = blockIdx.x % A.nsplit;
@@ -1161,6 +1206,7 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
   }
   const bool pen_on = wlen > 0 && (P0.repetition_penalty != 1.0 || P0.presence_penalty != 0.0 ||
                                    P0.frequency_penalty != 0.0);
+  const bool whole = !pen_on && whole_row(A, P0);
   if (pen_on && wlen > WIN_MAX) {                    // window longer than the LDS index
     if (t == 0) {
       my->flags = SF_UNSUPPORTED; my->ncand = 0; my->tau = 1u;
@@ -1191,6 +1237,27 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
   }
   __syncthreads();
   const cx_row_params& P = sP;
+  // a row drawn from whole (no filter, or typical-p alone): its chunks' sums
+  if (whole) {
+    if (t == 0) {
+      my->flags = SF_WHOLE; my->ncand = 0; my->tau = 1u; my->sxtol = 0;
+      my->m = 0; my->s = 0; my->tol = 0; my->sx = 0;
+      my->best_v = 0; my->best_i = INT_MAX; my->nan_i = INT_MAX;
+      if (split == 0) {
+        A.out_id[row] = -1;
+        A.row_status[row] = ROW_WHOLE;
+        A.counters[row] = ROW_WHOLE;
+      }
+    }
+    load_chunk<BF16>(rs, ch0 + NWAVE, qn);
+    if (!EXACT) {
+      if (t < 64) s_etab[t] = EXP64_TAB[t];
+      __syncthreads();
+    }
+    whole_slice<BF16>(whole_slice_of(A, split), rs, q, qn, nv, rowp, 1.0 / P.temperature, s_etab,
+                      (WholePart*)mycand);
+    return;
+  }
   // A single-slice bf16 row that may take the counted deep-nucleus path
   // (finish16_kernel counts its values, finding its maximum as it goes, and
   // decides it exactly or hands it to the exact path) is not streamed here:

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(WG) void slow_kernel(SampleArgs A) {
   __shared__ double red_d[2 * NWAVE + 4];
   __shared__ int red_i[2 * NWAVE + 4];
   __shared__ int s_state;
-  enum { DECIDED, MULTIPASS, REFINE, FINISH };
+  enum { DECIDED, MULTIPASS, REFINE, FINISH, WHOLE };
   const int row = (int)blockIdx.x;
   int state = FINISH;
   // a sliced row's status word is not written by the fused kernel: every
@@ -67,8 +67,9 @@ __global__ __launch_bounds__(WG) void slow_kernel(SampleArgs A) {
   if (A.pending_only || A.all_slow || A.nsplit == 1) {
     if (threadIdx.x == 0) {
       const int st = A.row_status[row];
-      s_state = A.pending_only ? (st == ROW_PENDING ? MULTIPASS : DECIDED)
-                : A.all_slow ? MULTIPASS
+      s_state = A.all_slow ? MULTIPASS
+                : st == ROW_WHOLE ? WHOLE
+                : A.pending_only ? (st == ROW_PENDING ? MULTIPASS : DECIDED)
                 : st == ROW_FINISH ? FINISH
                 : st == ROW_PENDING ? MULTIPASS
                 : st == ROW_REFINE ? REFINE : DECIDED;
@@ -81,12 +82,21 @@ __global__ __launch_bounds__(WG) void slow_kernel(SampleArgs A) {
     const cx_row_params P = A.prm[row];
     const int r = finish_row_fast<FIN_CAP>(A, row, P, dyn, red_d, red_i);
     if (r == FIN_DONE) return;
-    state = r == FIN_REFINE ? REFINE : MULTIPASS;
+    state = r == FIN_REFINE ? REFINE : r == FIN_WHOLE ? WHOLE : MULTIPASS;
     __syncthreads();
   }
-  if (state == REFINE && refine_row(A, row, dyn, red_d, red_i)) return;
-  __syncthreads();
-  if (deep_row(A, row, dyn, red_d, red_i)) return;
+  if (state == WHOLE) {
+    const cx_row_params P = A.prm[row];
+    WholeSums Z;
+    const int r = whole_finish(A, row, P, red_d, red_i, Z);
+    if (r == WHOLE_DONE) return;
+    __syncthreads();
+    if (r == WHOLE_TYP && deep_row(A, row, dyn, red_d, red_i, &Z)) return;
+  } else {
+    if (state == REFINE && refine_row(A, row, dyn, red_d, red_i)) return;
+    __syncthreads();
+    if (deep_row(A, row, dyn, red_d, red_i)) return;
+  }
   __syncthreads();
   slow_row(A, row, dyn, red_d, red_i);
 }
@@ -103,6 +113,7 @@ __device__ inline int f16_class(const SampleArgs& A, int row) {
   int m;
   if (A.nsplit > 1) {
     const cx_row_params& P = A.prm[row];
+    if (A.counters[row] == ROW_WHOLE) return 0;       // slow_kernel's
     m = ROW_FINISH | (deep_candidate(A, row, P, true) ? MARK_DEEP : 0) |
         (P.top_k > 0 && P.top_k < A.V ? MARK_TOPK : 0);
   } else {

@@ -216,3 +216,34 @@ def test_long_single_slice_rows_emulated():
         res = R.sample_row(c.logits, _params(c), c.hist, u, tie="spread")
         assert int(st[b]) & 0xFF == res.status, (c.name, int(st[b]), res.status)
         assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
+
+
+@pytest.mark.parametrize("V,nsplit", [(33000, None), (33001, None), (20003, "1")])
+def test_whole_rows_emulated(V, nsplit):
+    """Rows drawn from whole (no filter, or typical-p alone): sliced with
+    aligned rows, sliced with rows at odd addresses, and one slice; masked
+    (-inf) ids, a chunk of nothing else, and a coarse row whose equal values
+    straddle the typical cut.  The chunk records decide the unfiltered rows
+    (no exact path), the typical-order passes the typical-p ones."""
+    rng = np.random.default_rng(V)
+    base = dict(temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, typical_p=1.0,
+                repetition_penalty=1.0, n_keep=0)
+    rows = []
+    for i, kw in enumerate([dict(), dict(temperature=0.6), dict(typical_p=0.9),
+                            dict(typical_p=0.5, temperature=1.4), dict(typical_p=0.7)]):
+        x = rng.normal(0.0, 3.0, V).astype(np.float32)
+        if i in (1, 2):
+            x[rng.choice(V, V // 3, replace=False)] = -np.inf
+            x[2048:4096] = -np.inf
+        if i == 4:
+            x = np.round(x * 8) / 8
+        rows.append(cases.SamplerCase(f"whole{i}", x.astype(np.float32),
+                                      dict(base, **kw, seed=int(rng.integers(0, 2**31))), []))
+    with tempfile.TemporaryDirectory() as tmp:
+        (ids, st), = run_pipeline([rows], tmp, env={"EMU_NSPLIT": nsplit} if nsplit else None)
+    for b, c in enumerate(rows):
+        u = np.random.default_rng(c.params["seed"]).random()
+        res = R.sample_row(c.logits, _params(c), c.hist, u, tie="spread")
+        assert int(st[b]) & 0xFF == res.status, (c.name, int(st[b]), res.status)
+        assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
+        assert int(st[b]) >> 8 == (0 if c.params["typical_p"] == 1.0 else 0x5), (c.name, st[b])
