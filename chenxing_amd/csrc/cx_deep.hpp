@@ -39,9 +39,10 @@
 // exp per element, so no table entry can overflow.)
 //
 // Each thread reads 32 bytes per pass step (8 fp32 or 16 bf16 values).  On
-// 16-byte-aligned rows these are two range-checked buffer loads, issued
-// three steps ahead and unpacked only where used, so the loads stay in
-// flight; other rows load value by value.
+// rows that start at whole dwords (SampleArgs::vec_ok) these are two
+// range-checked buffer loads, issued three steps ahead and unpacked only
+// where used, so the loads stay in flight; bf16 rows at odd addresses load
+// value by value.
 //
 // Sums outside the histograms run in a fixed order in fp64.  Each term is
 // within 1 ulp, a bucket's integer sum within 2^-42 (relative) of its
@@ -278,7 +279,7 @@ __device__ __forceinline__ bool whole_row(const SampleArgs& A, const cx_row_para
 }
 
 // A slice's chunks: nvc of whole vectors from lo, then nsc over the rest
-// [s0, hi) (everything, on unaligned rows), 1024 ids each but the last of
+// [s0, hi) (everything, on bf16 rows at odd addresses), 1024 ids each but the last of
 // either kind.
 struct WholeSlice {
   int lo, s0, hi, nvc, nsc;
@@ -452,7 +453,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   R.step = R.nv * WG;
   R.p = (const char*)A.logits + (size_t)row * (size_t)A.ld * (R.bf16 ? 2 : 4);
   R.rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(R.p), (short)0,
-                                           (R.V * (R.bf16 ? 2 : 4) + 15) & ~15, 0x00020000);
+                                           (R.V * (R.bf16 ? 2 : 4) + 3) & ~3, 0x00020000);
   const int V = R.V, nv = R.nv;
   const double invT = 1.0 / P.temperature;
   const float Mf = (float)M, invTf = (float)invT;
@@ -853,7 +854,7 @@ __device__ inline double deep_exact_sum_impl(const SampleArgs& A, int row, doubl
   R.step = R.nv * WG;
   R.p = (const char*)A.logits + (size_t)row * (size_t)A.ld * (R.bf16 ? 2 : 4);
   R.rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(R.p), (short)0,
-                                           (R.V * (R.bf16 ? 2 : 4) + 15) & ~15, 0x00020000);
+                                           (R.V * (R.bf16 ? 2 : 4) + 3) & ~3, 0x00020000);
   const int t = threadIdx.x;
   // per step, the fetch's values as straight-line code (a loop bounded by
   // R.nv, with a break at hi, ran its exps one after another): four
@@ -892,7 +893,7 @@ __device__ inline double deep_exact_sum(const SampleArgs& A, int row, double M, 
 __device__ __forceinline__ bool deep_row(const SampleArgs& A, int row, unsigned char* dyn, double* red_d,
                                 int* red_i, const WholeSums* Z = nullptr) {
   const cx_row_params P = A.prm[row];
-  if (Z)             // (unaligned rows: the multi-pass path)
+  if (Z)             // (bf16 rows at odd addresses: the multi-pass path)
     return A.vec_ok && deep_row_impl<true, true>(A, row, P, Z->M, dyn, red_d, red_i, Z->c, Z->wt);
   double M = 0.0;
   if (!deep_eligible(A, row, P, M)) return false;

@@ -97,7 +97,7 @@ __device__ inline bool deep16_row_impl(const SampleArgs& A, int row, const cx_ro
   R.step = 16 * WG;
   R.p = (const char*)A.logits + (size_t)row * (size_t)A.ld * 2;
   R.rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(R.p), (short)0,
-                                           (R.V * 2 + 15) & ~15, 0x00020000);
+                                           (R.V * 2 + 3) & ~3, 0x00020000);
   const int V = R.V;
   const double invT = 1.0 / P.temperature;
   const int L = ((V + NWAVE * R.step - 1) / (NWAVE * R.step)) * R.step;
