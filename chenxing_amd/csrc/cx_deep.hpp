@@ -1,35 +1,40 @@
 // cx_deep.hpp -- rows whose nucleus is deeper than any region (reference
 // chenxing/core/sampler.py:81-93 and :117-127): top-p and min-p rows with no
 // top-k, no typical-p and no penalty window, which the fused kernel leaves
-// pending because their kept set outgrows its region.  One workgroup per
-// row; two passes over the row (three with min-p) and two short ones, in
-// place of the multi-pass path's eight or more:
+// pending because their kept set outgrows its region; and typical-p rows with
+// no other filter.  One workgroup per row; two passes over the row (three
+// with min-p) and two short ones, in place of the multi-pass path's eight or
+// more:
 //
-//   pass 1  every term e = exp((x - M) / T) <= 1 (M the row maximum the
-//           fused kernel found; table-driven fp64 exp): the row's sum S,
-//           and a histogram of e over DNB value buckets linear in
-//           (M - x) / T on [0, DSPAN).  A bucket sums its terms as integers
-//           in its own fixed-point scale (2^-F_b, F_b growing with the
-//           bucket's depth, so every term keeps about 42 significant bits and
-//           no sum overflows), so the sums do not depend on the order of the
-//           atomic additions.  At the end of each wave range (the row split
-//           into NWAVE contiguous id ranges) the histogram, summed into
-//           coarse buckets, is copied: the mass each range holds per coarse
-//           bucket.
-//   cut     the first bucket, from the top, whose running sum reaches
-//           top_p * S (sampler.py:82-85: cumsum of the sorted
-//           probabilities, searchsorted, one past the index)
-//   pass 2  the elements of that bucket, gathered, sorted by value
-//           (descending) and id (ascending) and scanned: the cut element;
-//           of the cut value's group the survivors spread over its ids
-//           (spread_kept, cx_device.hpp).  The same pass
-//           adds, per range, the terms of the cut's coarse bucket that lie
-//           above the cut bucket, so each range's kept mass follows from the
-//           copies.  (With min-p, pass 3 instead sums each range's kept terms
-//           again, testing e >= min_p per element, sampler.py:91-93.)
+//   pass 1  where the cut lies: a histogram of the terms exp((x - M) / T) (M
+//           the row maximum) over DNB value buckets linear in (M - x) / T on
+//           [0, DSPAN), the terms in fp32 rounded to integers of 12 bits or
+//           more in a scale of their bucket, and from it the buckets the
+//           running sum can reach top_p in, the roundings allowed for:
+//           usually one
+//   pass 2  in fp64, every term e = exp((x - M) / T) <= 1 (table-driven exp):
+//           the row's sum S and, per wave range (the row split into NWAVE
+//           contiguous id ranges), the sum above those buckets, in registers;
+//           the elements of the buckets themselves are gathered.
+//   cut     the gathered elements sorted by value (descending) and id
+//           (ascending) and scanned on from the sum above them
+//           (sampler.py:82-85: cumsum of the sorted probabilities,
+//           searchsorted, one past the index): the cut element; of the cut
+//           value's group the survivors spread over its ids (spread_kept,
+//           cx_device.hpp).  Each range's kept mass is its sum above plus its
+//           kept gathered elements.  (With min-p, pass 3 instead sums each
+//           range's kept terms again, testing e >= min_p per element,
+//           sampler.py:91-93.)
 //   draw    the range holding u * Z (Z the kept total), then its sixteenth
 //           (each wave sums one); one wave scans that sixteenth in id order
 //           (sampler.py:126-127: choice == searchsorted(cumsum, u, 'right'))
+//
+// Bound: pass 1 by the LDS additions (about 23 cycles a wave), pass 2 by the
+// fp64 VALU (a table exp per element), one CU per row.  An exact fixed-point
+// histogram in pass 1 instead (64-bit additions, per-range copies, and a
+// second pass that took another exponential for the elements between the
+// copies' boundary and the cut) took 59 + 46 us at V = 128256 fp32; fp32 LDS
+// additions in pass 1 take 164 us, eight times the 32-bit integer ones.
 //
 // On bf16 rows a term is the product of three LDS table entries, one per
 // part of the value's bits (sign, exponent and the top three mantissa bits;
@@ -44,13 +49,14 @@
 // where used, so the loads stay in flight; bf16 rows at odd addresses load
 // value by value.
 //
-// Sums outside the histograms run in a fixed order in fp64.  Each term is
-// within 1 ulp, a bucket's integer sum within 2^-42 (relative) of its
-// terms' sum, fp64 sums of at most 2^20 terms within 2^20 ulp, and the
-// reference's own cumulative sums within 4e-11 (relative) of exact: a
-// decision closer to its threshold than 5e-11 of the total returns false
-// and the row takes the multi-pass path, as do NaN rows, cuts below the
-// bucket span and cut buckets of more elements than the gather holds.
+// The sums that decide run in a fixed order in fp64 (but the kept gathered
+// terms, added as integers in units of 2^-51).  Each term is within 1 ulp
+// (2.5 ulp for the table product), fp64 sums of at most 2^20 terms within
+// 2^20 ulp, and the reference's own cumulative sums within 4e-11 (relative)
+// of exact: a decision closer to its threshold than 5e-11 of the total
+// returns false and the row takes the multi-pass path, as do NaN rows, cuts
+// below the bucket span and cut buckets of more elements than the gather
+// holds.
 #pragma once
 #include "cx_device.hpp"
 #include "cx_internal.hpp"
@@ -58,24 +64,22 @@
 namespace cx {
 
 constexpr int DNB = 4096;                     // value buckets
-constexpr int DCB = 64;                       // fine buckets per coarse bucket
-constexpr int DNCB = DNB / DCB;               // coarse buckets
 constexpr float DSPAN = 40.0f;                // bucket span below M, units of T (exp(-40) ~ 4e-18)
 constexpr float DSCALE = DNB / DSPAN;         // buckets per unit
-constexpr int DF0 = 42;                       // fixed-point bits of a term at its bucket's top
 constexpr double DTOL = 5e-11;                // relative decision margin
-constexpr int DCAP = 4 * WG;                  // cut-bucket capacity, fp32 rows (block_sort<4>)
-constexpr int DCAP16 = 2 * WG;                // cut-bucket capacity, bf16 rows
+constexpr int DCAP = 4 * WG;                  // gather capacity, fp32 rows (block_sort<4>)
+constexpr int DCAP16 = 2 * WG;                // gather capacity, bf16 rows
 constexpr int DW = 8;                         // 32-bit words per thread per step
 constexpr int DNV = 16;                       // most values per thread per step (bf16)
-// dynamic LDS: h[DNB] u64 | C[NWAVE][DNCB] f64 | X, where X holds the gather
-// (gk u64 | gi i32 | ga i32, DCAP entries) on fp32 rows and the three term
-// tables (4096 + 2048 + 2048 f64) on bf16 rows, whose gather (DCAP16
-// entries) reuses h once the cut bucket is known
-constexpr int DEEP_OFF_C = DNB * 8;
-constexpr int DEEP_OFF_X = DEEP_OFF_C + NWAVE * DNCB * 8;
+// dynamic LDS: h[2 DNB] u32 | ab[NWAVE][NWAVE] f64 | X, where X
+// holds the gather (gk u64 | gi i32 | ga i32, DCAP entries) on fp32 rows and
+// the three term tables (4096 + 2048 + 2048 f64) on bf16 rows, whose gather
+// (DCAP16 entries) takes h's place once the cut's buckets are known
+constexpr int DEEP_OFF_AB = DCAP16 * 16;
+constexpr int DEEP_OFF_X = DEEP_OFF_AB + NWAVE * NWAVE * 8;
 constexpr int DEEP_LDS = DEEP_OFF_X + DCAP * 16;
-static_assert(DCAP16 * 16 <= DNB * 8 && (4096 + 2048 + 2048) * 8 <= DCAP * 16, "deep LDS layout");
+static_assert(2 * DNB * 4 <= DEEP_OFF_AB && (4096 + 2048 + 2048) * 8 <= DCAP * 16 &&
+              DCAP16 >= 2 * WG, "deep LDS layout");
 
 // 16 bytes (vector_size, so host builds of this header compile too)
 typedef uint32_t deep_u32x4 __attribute__((vector_size(16)));
@@ -121,6 +125,14 @@ __device__ __forceinline__ void deep_fetch(const DeepRow& R, int e0, uint32_t (&
 __device__ __forceinline__ uint32_t deep_code(const uint32_t (&w)[DW], int j) {
   return (j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xFFFFu);
 }
+// Word j / 2 (bf16) or j (fp32) of a fetch for a j known only at run time:
+// selected, not indexed, so the fetch stays in registers.
+__device__ __forceinline__ uint32_t deep_word(const uint32_t (&w)[DW], int k) {
+  uint32_t r = 0u;
+#pragma unroll
+  for (int i = 0; i < DW; ++i) r |= k == i ? w[i] : 0u;
+  return r;
+}
 // Value j of a fetch.
 __device__ __forceinline__ float deep_val(const DeepRow& R, const uint32_t (&w)[DW], int j) {
   if (R.bf16) return __uint_as_float((j & 1) ? (w[j >> 1] & 0xFFFF0000u) : (w[j >> 1] << 16));
@@ -133,15 +145,6 @@ __device__ __forceinline__ float deep_val(const DeepRow& R, const uint32_t (&w)[
 __device__ __forceinline__ int deep_bucket(float x, float Mf, float invTf) {
   const float d = (Mf - x) * invTf;
   return d < DSPAN ? (int)(d * DSCALE) : -1;
-}
-// Fixed-point exponent of fine bucket b: its terms are at most
-// ~exp(-b / DSCALE) = 2^(-b * 0.0140888), so 2^(DF0 + floor(b * 923 / 2^16))
-// (923 / 2^16 = 0.0140839) keeps each term below 2^(DF0 + 1) and a sum of at
-// most 2^20 of them below 2^63.
-__device__ __forceinline__ int deep_scale(int b) { return DF0 + ((b * 923) >> 16); }
-// 2^e for |e| < 1023, from its bits
-__device__ __forceinline__ double deep_pow2(int e) {
-  return __longlong_as_double((long long)(1023 + e) << 52);
 }
 __device__ __forceinline__ double deep_term(float x, double M, double invT, const double* tab) {
   return exp64_neg(((double)x - M) * invT, tab);
@@ -193,6 +196,11 @@ __device__ __forceinline__ double block_excl_scan_d(double v, double* scratch) {
   __syncthreads();
   return r;
 }
+
+template <bool B>
+struct DeepFlag {
+  static constexpr bool value = B;
+};
 
 // f(k, w) for every step k < n of a pass over ids from lo on (this
 // thread's fetch w from id lo + k * stride + nv * idx on), with the next
@@ -336,8 +344,7 @@ constexpr int WHOLE_DONE = 1;      // drawn
 constexpr int WHOLE_TYP = 2;       // typical-p row: Z holds its sums for deep_row
 struct WholeSums {
   double M;          // row maximum
-  double c;          // -sum P d, d = (x - M) / T: the entropy less log S
-  double wt;         // 1 / sum exp(d)
+  double c;          // -sum P d, d = (x - M) / T: the entropy less log of sum exp(d)
 };
 
 // All threads of the workgroup; every thread gets the same result.  The
@@ -386,7 +393,6 @@ __device__ inline int whole_finish(const SampleArgs& A, int row, const cx_row_pa
   if (P.typical_p < 1.0) {
     Z.M = M;
     Z.c = -block_sum(dsum, red_d) / S;
-    Z.wt = 1.0 / S;
     return Z.c >= 0.0 ? WHOLE_TYP : WHOLE_OPEN;
   }
   // the chunk holding u * S (sampler.py:126-127), then the element in it
@@ -429,23 +435,23 @@ __device__ inline int whole_finish(const SampleArgs& A, int row, const cx_row_pa
 
 // TYP: a typical-p row with no other filter (sampler.py:95-105).  The same
 // passes in the typical order, ascending |d + c| with d = (x - M) / T and
-// c = -sum P d (whole_finish): the buckets are linear in that distance (in
-// fp64, so the two sides of the order compare exactly), the terms are the
-// probabilities e wt themselves, and a bucket sums them in units of 2^-60 (at
-// most 1 in all, so one scale serves every bucket).  A cut beside an element
-// of the other side whose distance differs by less than 1e-11 is left to
-// the multi-pass path.
+// c = -sum P d (whole_finish): the buckets are linear in that distance, in
+// fp64, so the two sides of the order compare exactly.  A cut beside an
+// element of the other side whose distance differs by less than 1e-11 is
+// left to the multi-pass path.
 template <bool VEC, bool TYP>
 __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, const cx_row_params& P,
                                      double M, unsigned char* dyn, double* red_d, int* red_i,
-                                     double c, double wt) {
+                                     double c) {
   __shared__ double tab[64];
   __shared__ double s_d[2 * NWAVE + 4];
   __shared__ double s_wm[NWAVE];                     // kept mass per wave range / sixteenth
-  __shared__ unsigned long long s_corr[2 * NWAVE];   // per range: cut coarse bucket, cut bucket
+  __shared__ unsigned long long s_kept[NWAVE];       // per range: the gathered kept terms
   __shared__ int s_i[4];
   __shared__ int s_g[2];
   const int t = threadIdx.x, l = lane_id(), w = wave_id();
+  M = lane_read(M, 0);                               // uniform: into scalar registers
+  c = lane_read(c, 0);
   DeepRow R;
   R.V = A.V;
   R.bf16 = A.bf16 != 0;
@@ -457,8 +463,8 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   const int V = R.V, nv = R.nv;
   const double invT = 1.0 / P.temperature;
   const float Mf = (float)M, invTf = (float)invT;
-  unsigned long long* h = (unsigned long long*)dyn;
-  double* C = (double*)(dyn + DEEP_OFF_C);          // C[r * DNCB + cb]: ranges 0..r, cumulative
+  uint32_t* h = (uint32_t*)dyn;                      // TYP: the upper side's from DNB on
+  double* ab = (double*)(dyn + DEEP_OFF_AB);         // ab[r * NWAVE + w]: range r's sum above, wave w's
   double* ta = (double*)(dyn + DEEP_OFF_X);
   double* tb = ta + 4096;
   double* tc = tb + 2048;
@@ -468,152 +474,192 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   unsigned char* gbase = R.bf16 ? dyn : dyn + DEEP_OFF_X;
   uint64_t* gk = (uint64_t*)gbase;
   int32_t* gi = (int32_t*)(gbase + cap * 8);
-  int32_t* ga = (int32_t*)(gbase + cap * 12);
+  int32_t* ga = (int32_t*)(gbase + cap * 12);        // the value's bits
   // wave ranges: NWAVE contiguous id ranges of L ids, L a multiple of the
   // step, so each workgroup step lies in one range
   const int L = ((V + NWAVE * R.step - 1) / (NWAVE * R.step)) * R.step;
-  const int nsteps = (V + R.step - 1) / R.step;
-  // the typical order's distance of value x, its bucket (-1 past the span),
-  // and the fixed-point scale of a bucket's terms
+  const int nsteps = (V + R.step - 1) / R.step, spr = L / R.step;
+  int range = 0, left = spr;                         // pass 2's range, and its steps left
+  // the typical order's distance of value x; the bucket of x (-1 past the
+  // span): the same expression in every pass
   auto dist = [&](float x) { return fabs(((double)x - M) * invT + c); };
   auto bucket = [&](float x) -> int {
     if constexpr (!TYP) return deep_bucket(x, Mf, invTf);
     const double v = dist(x) * (double)DSCALE;
     return v < (double)DNB ? (int)v : -1;
   };
-  auto scale = [&](int b) { return deep_pow2(TYP ? 60 : deep_scale(b)); };
-  auto unscale = [&](int b) { return deep_pow2(TYP ? -60 : -deep_scale(b)); };
-  auto term = [&](float x) { return TYP ? deep_term(x, M, invT, tab) * wt : deep_term(x, M, invT, tab); };
-  auto term16 = [&](uint32_t code) {
-    return TYP ? deep_term16(code, ta, tb, tc) * wt : deep_term16(code, ta, tb, tc);
+  // pass 1's integers have wbits bits, as many as keep V of them below 2^32:
+  // 2^s brings the bucket's largest term (of the typical order's upper side,
+  // d + c > 0, where the terms grow with the distance) just below 2^wbits.
+  // A bucket's sum is then within 2^-wbits of its terms' (fp32 terms: 1e-5).
+  const int wbits = __clz(V);
+  const double eps = __builtin_ldexp(1.0, -wbits) + 1e-5;
+  constexpr float LOG2E = 1.44269504f;
+  const float cf = (float)c;
+  auto weight_scale = [&](int b, bool up) -> int {
+    const float top = up ? (float)(b + 1) * (1.0f / DSCALE) - cf : (float)b * (-1.0f / DSCALE) - cf;
+    return wbits - 1 - (int)__builtin_ceilf(top * LOG2E);
   };
-  for (int b = t; b < DNB; b += WG) h[b] = 0ull;
-  if (t < 2 * NWAVE) s_corr[t] = 0ull;
+  const bool cut = TYP || P.top_p < 1.0;
+  // (a typical target so small that 2^-51 units no longer resolve it)
+  if (TYP && !(P.typical_p >= 0.02)) return false;
+  // (bf16 rows at odd addresses have the term-table pass only)
+  if (!VEC && !use_tab) return false;
+  for (int b = t; b < 2 * DNB; b += WG) h[b] = 0u;
+  for (int b = t; b < NWAVE * NWAVE; b += WG) ab[b] = 0.0;
+  if (t < NWAVE) s_kept[t] = 0ull;
   if (t == 0) s_i[0] = 0;
   load_exp64_tab(tab);                               // its barrier also orders the clears
-  if (use_tab) {
-    deep_build_tables(ta, tb, tc, M, invT, tab);
-    __syncthreads();
-  }
 
-  // ---- pass 1: S and the bucket histograms, copied at each range's end
-  double s = 0.0;
-  int bad = 0;
-  deep_stream<VEC>(R, 0, R.step, t, nsteps, [&](int k, const uint32_t (&wd)[DW]) {
-    const int e0 = k * R.step + nv * t;
-#pragma unroll
-    for (int j = 0; j < DNV; ++j) {
-      if (j >= nv || e0 + j >= V) break;
-      const float x = deep_val(R, wd, j);
-      if (!(x == x) || x > Mf) { bad = 1; continue; }
-      const int b = bucket(x);
-      // (the tables leave out terms below the span: at most V exp(-40) in all)
-      const double ev = !use_tab ? term(x) : (b >= 0 ? term16(deep_code(wd, j)) : 0.0);
-      s += ev;
-      if (b >= 0) atomicAdd(h + b, (unsigned long long)(ev * scale(b)));
-    }
-    const int r = (k * R.step) / L;
-    if ((k + 1) * R.step % L == 0 || k + 1 == nsteps) {
-      // the histogram so far, summed into coarse buckets (16 threads each)
-      __syncthreads();
-      double v = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v += (double)h[4 * t + j] * unscale(4 * t + j);
-      v = row_reduce(v, OpAdd());
-      for (int rr = r; rr < (k + 1 == nsteps ? NWAVE : r + 1); ++rr)
-        if ((t & 15) == 0) C[rr * DNCB + (t >> 4)] = v;
-      __syncthreads();
-    }
-  });
-  const double S = block_sum(s, s_d);
-  if (block_max(bad, red_i, 0)) return false;        // NaN (or a value above M)
-  const double tolS = DTOL * S;
-
-  // ---- the cut: first non-empty bucket whose inclusive sum reaches top_p * S
-  const bool cut = TYP || P.top_p < 1.0;
-  float xcut = -__builtin_inff();
-  double dcut = 0.0;                                 // TYP: the cut distance
-  int g0 = 0, gn = 0, gj = 0;                        // the cut value's group: none
-  int bs = DNB;                                      // no cut: every bucket above it
+  // ---- pass 1: the buckets [blo, bhi] that hold the cut
+  int blo = DNB, bhi = DNB;                          // no cut: every bucket above it
   if (cut) {
-    const double tgt = (TYP ? P.typical_p : P.top_p) * S;
-    double vb[4];
-    double c4 = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      vb[j] = (double)h[4 * t + j] * unscale(4 * t + j);
-      c4 += vb[j];
-    }
-    double before = block_excl_scan_d(c4, s_d);
-    int bstar = INT_MAX;
-    double above = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const double incl = before + vb[j];
-      if (bstar == INT_MAX && h[4 * t + j] != 0ull && incl >= tgt) {
-        bstar = 4 * t + j;
-        above = before;
-      }
-      before = incl;
-    }
-    bs = block_min(bstar, red_i, INT_MAX);
-    if (bs == INT_MAX) return false;                 // the cut lies below the span
-    if (bstar == bs) red_d[2 * NWAVE + 2] = above;
-    __syncthreads();
-    above = red_d[2 * NWAVE + 2];
-    __syncthreads();
-
-    // ---- pass 2: gather the cut bucket; per range, the terms of the cut's
-    // coarse bucket above it (the copies end at coarse-bucket boundaries)
-    const bool corr = P.min_p <= 0.0;
-    const int cb0 = (bs / DCB) * DCB;
-    const double fc = scale(cb0);
-    unsigned long long acc = 0ull;
     deep_stream<VEC>(R, 0, R.step, t, nsteps, [&](int k, const uint32_t (&wd)[DW]) {
       const int e0 = k * R.step + nv * t;
 #pragma unroll
       for (int j = 0; j < DNV; ++j) {
         if (j >= nv) break;
-        const float x = deep_val(R, wd, j);
-        const int b = e0 + j < V ? bucket(x) : -1;
-        // the cut bucket's elements, placed by one LDS atomic per wave
-        const bool g = b == bs;
-        const uint64_t m = ballot(g);
-        if (m) {
-          int base = 0;
-          if (l == 0) base = atomicAdd(s_i, __popcll(m));
-          base = __builtin_amdgcn_readfirstlane(base);
-          const int pos = base + lanes_below(m);
-          if (g && pos < cap) {
-            gk[pos] = d2key(TYP ? -dist(x) : (double)x);
-            gi[pos] = e0 + j;
-            ga[pos] = (int32_t)__float_as_uint(x);
-          }
-        }
-        if (corr && b >= cb0 && b < bs)
-          acc += (unsigned long long)((use_tab ? term16(deep_code(wd, j)) : term(x)) * fc);
-      }
-      if (corr && ((k + 1) * R.step % L == 0 || k + 1 == nsteps)) {
-        const unsigned long long m = wave_sum(acc);
-        if (l == 0 && m != 0ull) atomicAdd(s_corr + (k * R.step) / L, m);
-        acc = 0ull;
+        const float x = e0 + j < V ? deep_val(R, wd, j) : -__builtin_inff();
+        const int b = bucket(x);
+        const bool up = TYP && ((double)x - M) * invT + c > 0.0;
+        const float lg = (x - Mf) * invTf * LOG2E + (float)weight_scale(b, up);
+        if (b >= 0)
+          atomicAdd(h + (up ? DNB : 0) + b, (uint32_t)(__builtin_amdgcn_exp2f(lg) + 0.5f));
       }
     });
     __syncthreads();
-    const int ng = s_i[0];
+    double vb[4];
+    double c4 = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int b = 4 * t + j;
+      vb[j] = __builtin_ldexp((double)h[b], -weight_scale(b, false));
+      if (TYP) vb[j] += __builtin_ldexp((double)h[DNB + b], -weight_scale(b, true));
+      c4 += vb[j];
+    }
+    const double Sa = block_sum(c4, s_d);
+    const double p = TYP ? P.typical_p : P.top_p;
+    double incl = block_excl_scan_d(c4, s_d);
+    int b0 = INT_MAX, b1 = INT_MAX;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      incl += vb[j];
+      if (b0 == INT_MAX && vb[j] != 0.0 && incl >= (p - eps) * Sa) b0 = 4 * t + j;
+      if (b1 == INT_MAX && vb[j] != 0.0 && incl >= (p + eps) * Sa) b1 = 4 * t + j;
+    }
+    // (uniform values, here and below, into scalar registers)
+    blo = __builtin_amdgcn_readfirstlane(block_min(b0, red_i, INT_MAX));
+    bhi = __builtin_amdgcn_readfirstlane(min(block_min(b1, red_i, INT_MAX), DNB - 1));
+    if (blo == INT_MAX) return false;                // NaN sums
+  }
+  if (use_tab) {
+    deep_build_tables(ta, tb, tc, M, invT, tab);
     __syncthreads();
-    if (ng > cap) return false;
-    block_sort<4>(gk, gi, ga, ng);                   // key descending, id ascending
+  }
+
+  // ---- pass 2: S, the sums above the cut's buckets, and their elements
+  double s = 0.0, above = 0.0;
+  int bad = 0;
+  auto pass2 = [&](auto tables) __attribute__((always_inline)) {
+  deep_stream<VEC>(R, 0, R.step, t, nsteps, [&](int k, const uint32_t (&wd)[DW]) {
+    constexpr bool TAB = decltype(tables)::value;
+    const int e0 = k * R.step + nv * t;
+    uint32_t mg = 0u;
+#pragma unroll
+    for (int j = 0; j < DNV; ++j) {
+      if (j >= nv) break;
+      const float x = e0 + j < V ? deep_val(R, wd, j) : -__builtin_inff();
+      const int b = bucket(x);
+      // (the tables leave out terms below the span: at most V exp(-40) in all)
+      const double e = !TAB ? deep_term(x, M, invT, tab)
+                            : (b >= 0 ? deep_term16(deep_code(wd, j), ta, tb, tc) : 0.0);
+      if (!(x <= Mf)) bad = 1;
+      s += e;
+      above += (uint32_t)b < (uint32_t)blo ? e : 0.0;
+      if ((uint32_t)(b - blo) <= (uint32_t)(bhi - blo)) mg |= 1u << j;
+      // the sums so far: left to the end of the step, the selects keep every
+      // term of it in a register
+      if ((j & 3) == 3) __asm__ volatile("" : "+v"(s), "+v"(above), "+v"(mg), "+v"(bad));
+    }
+    // the lane's elements of the cut's buckets, one by one (few lanes have any)
+    while (mg) {
+      const int j = __builtin_ctz(mg);
+      mg &= mg - 1u;
+      const uint32_t wj = deep_word(wd, R.bf16 ? j >> 1 : j);
+      const float x = __uint_as_float(!R.bf16 ? wj : (j & 1) ? (wj & 0xFFFF0000u) : (wj << 16));
+      const int pos = atomicAdd(s_i, 1);
+      if (pos < cap) {
+        gk[pos] = d2key(TYP ? -dist(x) : (double)x);
+        gi[pos] = e0 + j;
+        ga[pos] = (int32_t)__float_as_uint(x);
+      }
+    }
+    if (--left == 0 || k + 1 == nsteps) {
+      const double m = wave_reduce(above, OpAdd());
+      if (l == 0) ab[range * NWAVE + w] = m;
+      above = 0.0;
+      ++range;
+      left = spr;
+    }
+  });
+  };
+  // (a branch per element would leave each wave waiting for its own table
+  // read: 51 us at V = 128256 fp32)
+  if (use_tab) pass2(DeepFlag<true>());
+  else if constexpr (VEC) pass2(DeepFlag<false>());
+  const double S = lane_read(block_sum(s, s_d), 0);
+  if (block_max(bad, red_i, 0)) return false;        // NaN (or a value above M)
+  const double tolS = DTOL * S;
+
+  float xcut = -__builtin_inff();
+  double dcut = 0.0;                                 // TYP: the cut distance
+  int g0 = 0, gn = 0, gj = 0;                        // the cut value's group: none
+  if (cut) {
+    const double tgt = (TYP ? P.typical_p : P.top_p) * S;
+    const double total = lane_read(block_sum(t < NWAVE * NWAVE ? ab[t] : 0.0, s_d), 0);
+    const int ng = __builtin_amdgcn_readfirstlane(s_i[0]);
+    __syncthreads();
+    if (ng > cap || ng == 0) return false;
+    // key descending, id ascending: up to one entry per thread (the usual
+    // case: a few hundred) by counting the entries before each, the count
+    // split over the threads left (the bitonic sort takes 14 us)
+    if (ng <= WG) {
+      int* rank = (int*)(gk + WG);
+      const int np = max(64, 1 << (32 - __clz(max(ng, 2) - 1)));
+      const int parts = WG / np, e = t & (np - 1), pt = t / np;
+      rank[t] = 0;
+      __syncthreads();
+      const uint64_t ke = e < ng ? gk[e] : 0ull;
+      const int32_t ie = e < ng ? gi[e] : 0, ae = e < ng ? ga[e] : 0;
+      const int j0 = pt * ng / parts, j1 = (pt + 1) * ng / parts;
+      int before = 0, same = e >= j0 && e < j1 ? -1 : 0;
+#pragma unroll 4
+      for (int j = j0; j < j1; ++j) {
+        const uint64_t kj = gk[j];
+        before += kj > ke ? 1 : 0;
+        same += kj == ke ? 1 : 0;
+      }
+      // equal keys by id (fp32 rows: hardly ever any)
+      if (ballot(e < ng && same > 0))
+        for (int j = j0; j < j1; ++j) before += gk[j] == ke && gi[j] < ie ? 1 : 0;
+      if (e < ng && before > 0) atomicAdd(rank + e, before);
+      __syncthreads();
+      const int re = rank[e];
+      if (pt == 0 && e < ng) { gk[re] = ke; gi[re] = ie; ga[re] = ae; }
+      __syncthreads();
+    } else {
+      block_sort<4>(gk, gi, ga, ng);
+    }
     // thread t: sorted entries 4t .. 4t+3, their terms and running sums
     double qv[4];
     double s4 = 0.0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e = 4 * t + j;
-      qv[j] = e < ng ? term(__uint_as_float((uint32_t)ga[e])) : 0.0;
+      qv[j] = e < ng ? deep_term(__uint_as_float((uint32_t)ga[e]), M, invT, tab) : 0.0;
       s4 += qv[j];
     }
-    double run = above + block_excl_scan_d(s4, s_d);
+    double run = total + block_excl_scan_d(s4, s_d);
     int jstar = INT_MAX;
     double cprev = 0.0, cstar = 0.0;
 #pragma unroll
@@ -627,12 +673,12 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       }
       run = incl;
     }
-    const int js = block_min(jstar, red_i, INT_MAX);
+    const int js = __builtin_amdgcn_readfirstlane(block_min(jstar, red_i, INT_MAX));
     if (js == INT_MAX) return false;
     if (jstar == js) {
       // robust: this element's running sum clearly reaches the target and
       // the one before clearly does not (the first element is always kept)
-      const bool first = !TYP && bs == 0 && js == 0;
+      const bool first = !TYP && total == 0.0 && js == 0;
       const bool ok = cstar >= tgt + tolS && (first || cprev < tgt - tolS);
       s_i[1] = ok ? 1 : 0;
       s_g[0] = js;
@@ -665,21 +711,18 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       __syncthreads();
       if (!s_i[1]) return false;
     }
-    if constexpr (TYP) dcut = -red_d[2 * NWAVE + 2];
-    else xcut = (float)red_d[2 * NWAVE + 2];
-    g0 = s_g[0];
-    gn = s_g[1] - g0;
+    if constexpr (TYP) dcut = lane_read(-red_d[2 * NWAVE + 2], 0);
+    else xcut = (float)lane_read(red_d[2 * NWAVE + 2], 0);
+    g0 = __builtin_amdgcn_readfirstlane(s_g[0]);
+    gn = __builtin_amdgcn_readfirstlane(s_g[1]) - g0;
     gj = js + 1 - g0;
-    // the kept part of the cut bucket, per range: the entries above the cut
-    // value and the group's survivors
-    if (corr) {
-      const double fb = scale(bs);
+    // the kept part of the gathered elements, per range: the entries above
+    // the cut value and the group's survivors
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int e = 4 * t + j;
-        if (e < g0 || (e < g0 + gn && spread_keeps(e - g0, gj, gn, V <= TIE_NET)))
-          atomicAdd(s_corr + NWAVE + gi[e] / L, (unsigned long long)(qv[j] * fb));
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int e = 4 * t + j;
+      if (e < g0 || (e < g0 + gn && spread_keeps(e - g0, gj, gn, V <= TIE_NET)))
+        atomicAdd(s_kept + gi[e] / L, (unsigned long long)(qv[j] * 2251799813685248.0));
     }
     __syncthreads();
   }
@@ -707,7 +750,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
       const uint32_t kx = f2key(x);
       if (!(kx > kcut || (kx == kcut && in_group(id)))) return 0.0;
     }
-    const double ev = term(x);
+    const double ev = deep_term(x, M, invT, tab);
     if (minp > 0.0) {
       if (fabs(ev - minp) <= minp_tol) amb = 1;
       if (ev < minp) return 0.0;
@@ -731,18 +774,12 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     return wave_sum(m);
   };
 
-  // ---- each range's kept mass: from the copies (no min-p), or pass 3
+  // ---- each range's kept mass: its sums above the cut's buckets and its
+  // kept gathered terms (no min-p), or pass 3
   if (minp <= 0.0) {
-    if (t < NWAVE) {
-      const int cbs = cut ? bs / DCB : DNCB;          // coarse buckets wholly kept
-      double m = 0.0;
-      for (int cb = 0; cb < cbs; ++cb)
-        m += C[t * DNCB + cb] - (t > 0 ? C[(t - 1) * DNCB + cb] : 0.0);
-      if (cut)
-        m += (double)s_corr[t] * unscale((bs / DCB) * DCB) +
-             (double)s_corr[NWAVE + t] * unscale(bs);
-      s_wm[t] = m;
-    }
+    double m = l < NWAVE ? ab[w * NWAVE + l] : 0.0;
+    m = wave_reduce(m, OpAdd());
+    if (l == 0) s_wm[w] = m + (double)s_kept[w] * 4.440892098500626e-16;   // 2^-51
     __syncthreads();
   } else {
     const double m = wave_mass(w * L, w * L + L);
@@ -753,7 +790,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   for (int k = 0; k < NWAVE; ++k) Z += s_wm[k];
   if (!(Z > 0.0)) return false;
   const double tolZ = DTOL * Z;
-  const double t2 = A.u[row] * Z;
+  const double t2 = lane_read(A.u[row] * Z, 0);
   // the wave range holding t2
   int wr = -1;
   double off = 0.0;
@@ -894,11 +931,11 @@ __device__ __forceinline__ bool deep_row(const SampleArgs& A, int row, unsigned 
                                 int* red_i, const WholeSums* Z = nullptr) {
   const cx_row_params P = A.prm[row];
   if (Z)             // (bf16 rows at odd addresses: the multi-pass path)
-    return A.vec_ok && deep_row_impl<true, true>(A, row, P, Z->M, dyn, red_d, red_i, Z->c, Z->wt);
+    return A.vec_ok && deep_row_impl<true, true>(A, row, P, Z->M, dyn, red_d, red_i, Z->c);
   double M = 0.0;
   if (!deep_eligible(A, row, P, M)) return false;
-  return A.vec_ok ? deep_row_impl<true, false>(A, row, P, M, dyn, red_d, red_i, 0.0, 1.0)
-                  : deep_row_impl<false, false>(A, row, P, M, dyn, red_d, red_i, 0.0, 1.0);
+  return A.vec_ok ? deep_row_impl<true, false>(A, row, P, M, dyn, red_d, red_i, 0.0)
+                  : deep_row_impl<false, false>(A, row, P, M, dyn, red_d, red_i, 0.0);
 }
 
 }  // namespace cx
