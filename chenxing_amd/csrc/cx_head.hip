@@ -87,8 +87,8 @@ __device__ __forceinline__ uint64_t head_key(float x, int v) {
 //    D = 4096: B = 32 213 -> 189 us, B = 64 228 -> 195 us (with rows padded
 //    by 128 bytes: 184 and 195 us); two starts instead of four give nothing,
 //    and for larger batches four sets of accumulators do not fit.
-//  * Measured, B = 256, V = 128256, D = 4096: 305 us, 880 TFLOP/s (1436 us with
-//    32 batch rows per pass over the weights); B = 128 246 us (was 757 us);
+//  * Measured, B = 256, V = 128256, D = 4096: 291 us, 925 TFLOP/s (1416 us with
+//    32 batch rows per pass over the weights); B = 128 241 us (was 757 us);
 //    B = 16, V = 32000 50 us (131 us with 512 vocab rows a workgroup, which
 //    left 193 of the 256 CUs without one).
 constexpr int WIDE_SK = 64;                  // k per stage
@@ -174,18 +174,27 @@ __global__ __launch_bounds__(NW * 64, 1) void head_wide(HeadArgs A) {
   // this lane's operand chunk in a stage buffer: row c of tile 0, slice 0
   const int lofs = c * WIDE_SK + 8 * (g ^ (c & 7));
   auto multiply = [&](const uint16_t* buf, const WideStage<MT>& x, f32x4 (&acc)[MT][NT]) {
+    // four operand reads ahead of their MFMAs, kept in that order (two reads
+    // and a wait, as the scheduler places them: 303 instead of 291 us at
+    // B = 256, V = 128256, D = 4096)
+    constexpr int OPS = 2 * NT, AHEAD = 4;
+    auto operand = [&](int i) {
+      return *(const CX_LDS u32x4*)(to_lds((uint16_t*)buf) + (lofs ^ (32 * (i / NT))) +
+                                    (i % NT) * 16 * WIDE_SK);
+    };
+    u32x4 h[AHEAD];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int i = 0; i < AHEAD; ++i) h[i] = operand(i);
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const u32x4 h = *(const CX_LDS u32x4*)(to_lds((uint16_t*)buf) + (lofs ^ (32 * t)) +
-                                               n * 16 * WIDE_SK);
+    for (int i = 0; i < OPS; ++i) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, x.w[m][t]), __builtin_bit_cast(bf16x8, h), acc[m][n],
-              0, 0, 0);
-      }
+      for (int m = 0; m < MT; ++m)
+        acc[m][i % NT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, x.w[m][i / NT]), __builtin_bit_cast(bf16x8, h[i % AHEAD]),
+            acc[m][i % NT], 0, 0, 0);
+      if (i + AHEAD < OPS) h[i % AHEAD] = operand(i + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
   // Stage s has arrived once at most the later stages' loads are outstanding.
   auto step = [&](int s, uint16_t* cur, const WideStage<MT>& x, uint16_t* nxt, WideStage<MT>& y,

@@ -22,6 +22,9 @@
 //   * greedy rows: the first argmax over the unpenalised elements (a bitmap
 //     test per vector), merged with the penalised values afterwards.
 //
+//   * rows drawn from whole (no top-k, top-p or min-p, no penalty window):
+//     per 1024 elements the maximum and the fp64 sums against it.
+//
 // Top-k rows with one slice and a small region are decided in the same
 // workgroup by one wave.  Every other row writes its region and statistics
 // (one record per slice) and is finished by slow_kernel (cx_slow.hip), the

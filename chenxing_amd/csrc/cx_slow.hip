@@ -10,7 +10,9 @@
 //                     multi-pass path, as does any row the steps before
 //                     cannot decide; a pending top-p / min-p row without
 //                     top-k, typical-p or penalties first tries the
-//                     bucketed deep-nucleus path (cx_deep.hpp).  A
+//                     bucketed deep-nucleus path (cx_deep.hpp); rows drawn
+//                     from whole are drawn from the fused kernel's chunk
+//                     sums there (typical-p: the same passes).  A
 //                     workgroup whose row is decided reads its status word
 //                     and exits.  In a bf16 call it takes only the rows
 //                     finish16_kernel hands back.
