@@ -283,7 +283,7 @@ static_assert((SLICE_MAX / WCH + 2) * sizeof(WholePart) <= CAPS * sizeof(Cand),
 // (a row without a penalty window; ln V / T > 740: P**(1/T) may underflow)
 __device__ __forceinline__ bool whole_row(const SampleArgs& A, const cx_row_params& P) {
   return !(P.top_k > 0 && P.top_k < A.V) && !(P.top_p < 1.0) && !(P.min_p > 0.0) &&
-         P.temperature > 0.0 && !A.out_probs && A.logV * (1.0 / P.temperature) <= 740.0;
+         P.temperature > 0.0 && !A.out_probs && A.logV <= 740.0 * P.temperature;
 }
 
 // A slice's chunks: nvc of whole vectors from lo, then nsc over the rest

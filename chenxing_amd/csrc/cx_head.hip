@@ -88,7 +88,7 @@ __device__ __forceinline__ uint64_t head_key(float x, int v) {
 //    by 128 bytes: 184 and 195 us); two starts instead of four give nothing,
 //    and for larger batches four sets of accumulators do not fit.
 //  * Measured, B = 256, V = 128256, D = 4096: 291 us, 925 TFLOP/s (1416 us with
-//    32 batch rows per pass over the weights); B = 128 241 us (was 757 us);
+//    32 batch rows per pass over the weights); B = 128 241 us (was 704 us);
 //    B = 16, V = 32000 50 us (131 us with 512 vocab rows a workgroup, which
 //    left 193 of the 256 CUs without one).
 constexpr int WIDE_SK = 64;                  // k per stage

@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
   __syncthreads();
   const cx_row_params& P = sP;
   // a row drawn from whole (no filter, or typical-p alone): its chunks' sums
-  if (whole) {
+  if (__builtin_expect(whole, 0)) {
     if (t == 0) {
       my->flags = SF_WHOLE; my->ncand = 0; my->tau = 1u; my->sxtol = 0;
       my->m = 0; my->s = 0; my->tol = 0; my->sx = 0;

@@ -225,7 +225,10 @@ namespace emu {
 // the dynamic LDS of the workgroup being run: an exact-size allocation of
 // the bytes its launch requests
 extern unsigned char* dyn_lds;
+// the arguments of the kernel being run
+extern const void* kernarg;
 }  // namespace emu
+inline const void* __builtin_amdgcn_kernarg_segment_ptr() { return emu::kernarg; }
 typedef void* hipStream_t;
 #include <algorithm>
 using std::min;

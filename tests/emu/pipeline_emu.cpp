@@ -41,6 +41,7 @@ void emu::check_sites(int wi) {
   if (me == bad) _exit(4);
 }
 unsigned char* emu::dyn_lds;
+const void* emu::kernarg;
 using namespace cx;
 
 namespace cx {
@@ -122,6 +123,7 @@ static void run_workgroup(K kernel, const SampleArgs& A, unsigned block, size_t 
   unsigned char* dyn = (unsigned char*)malloc(lds > 0 ? lds : 1);
   for (size_t i = 0; i < lds; ++i) dyn[i] = (unsigned char)(i * 131 + 7 + block);
   emu::dyn_lds = dyn;
+  emu::kernarg = &A;
   emu::Wave waves[16];
   emu::waves = waves;
   std::barrier<> bb(1024);
