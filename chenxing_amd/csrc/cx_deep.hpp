@@ -509,7 +509,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   for (int b = t; b < 2 * DNB; b += WG) h[b] = 0u;
   for (int b = t; b < NWAVE * NWAVE; b += WG) ab[b] = 0.0;
   if (t < NWAVE) s_kept[t] = 0ull;
-  if (t == 0) s_i[0] = 0;
+  if (t == 0) { s_i[0] = 0; s_i[2] = 0; }
   load_exp64_tab(tab);                               // its barrier also orders the clears
 
   // ---- pass 1: the buckets [blo, bhi] that hold the cut
@@ -691,12 +691,15 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     // the cut value's group: sorted positions [g0, g1), ascending ids
     {
       const uint64_t kj = gk[js];
+      auto diff = [&](int e) { return (double)__uint_as_float((uint32_t)ga[e]) - M; };
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int e = 4 * t + j;
         if (e < ng && gk[e] == kj) { atomicMin(&s_g[0], e); atomicMax(&s_g[1], e + 1); }
-        // (the order's other side at the very same distance)
-        if (TYP && e < ng && gk[e] == kj && ga[e] != ga[js]) s_i[1] = 0;
+        // another d at the very same distance, the order's other side as a
+        // rule (+0 and -0, or values that x - M rounds together, are one d;
+        // its own flag, since waves behind this one still read s_i[1] above)
+        if (TYP && e < ng && gk[e] == kj && diff(e) != diff(js)) s_i[2] = 1;
       }
     }
     __syncthreads();
@@ -707,7 +710,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
         const bool near = (s_g[0] > 0 && key2d(gk[s_g[0] - 1]) - kd < 1e-11) ||
                           (s_g[1] < ng && kd - key2d(gk[s_g[1]]) < 1e-11) ||
                           fabs(fr - __builtin_rint(fr)) < 1e-8;   // beside the next bucket
-        if (near) s_i[1] = 0;
+        if (near || s_i[2]) s_i[1] = 0;
       }
       __syncthreads();
       if (!s_i[1]) return false;

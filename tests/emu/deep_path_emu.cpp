@@ -2,8 +2,10 @@
 // Runs a deep-nucleus row path on the host (deep_row, cx_deep.hpp, or with
 // MODE 16 deep16_row, cx_deep16.hpp), one workgroup at a time, with every
 // buffer an exact-size heap allocation under AddressSanitizer.  Each row's
-// maximum goes into its slice record, as the fused kernel leaves it.  Output
-// per row: the sampled id, or -2 where the path hands the row back.
+// maximum goes into its slice record, as the fused kernel leaves it; a
+// typical-p row gets its entropy shift c from the input, or, where that is
+// NaN, computed as whole_finish does.  Output per row: the sampled id, or -2
+// where the path hands the row back.
 // usage: deep_path_emu IN OUT [MODE] (written and read by tests/test_emu_deep_path.py)
 #include "cx_deep16.hpp"
 thread_local EmuDim threadIdx;
@@ -53,6 +55,7 @@ int main(int argc, char** argv) {
     void* x = rd<unsigned char>(in, (size_t)B * V * esz);
     cx_row_params* prm = rd<cx_row_params>(in, B);
     double* u = rd<double>(in, B);
+    double* c = rd<double>(in, B);
     int32_t* ids = (int32_t*)malloc(4 * B);
     int32_t* st = (int32_t*)malloc(4 * B);
     SplitStats* stats = (SplitStats*)calloc(B, sizeof(SplitStats));
@@ -85,6 +88,19 @@ int main(int argc, char** argv) {
       emu::block_bar = &bb;
       blockIdx.x = row;
       int decided = -1;
+      const bool typ = prm[row].typical_p < 1.0;
+      WholeSums Z{maxes[row], c[row]};
+      if (typ && std::isnan(Z.c)) {
+        double sp = 0.0, spd = 0.0;
+        for (int i = 0; i < V; ++i) {
+          const float v = bf16 ? __uint_as_float((uint32_t)((const uint16_t*)x)[(size_t)row * V + i] << 16)
+                               : ((const float*)x)[(size_t)row * V + i];
+          const double d = std::max(((double)v - Z.M) / prm[row].temperature, -745.2);
+          sp += exp(d);
+          spd += exp(d) * d;
+        }
+        Z.c = -spd / sp;
+      }
       std::vector<std::thread> th;
       th.reserve(1024);
       for (int t = 0; t < 1024; ++t)
@@ -94,7 +110,8 @@ int main(int argc, char** argv) {
           __shared__ int red_i[2 * NWAVE + 4];
           __shared__ Deep16Shared sh;
           const bool r = counted ? deep16_row(A, row, dyn, red_d, red_i, sh)
-                                 : deep_row(A, row, dyn, red_d, red_i);
+                                 : deep_row(A, row, dyn, red_d, red_i, typ ? &Z : nullptr);
+          emu::leave();
           if (t == 0) decided = r ? 1 : 0;
           waves[t >> 6].bar.arrive_and_drop();
           bb.arrive_and_drop();
@@ -111,7 +128,7 @@ int main(int argc, char** argv) {
     }
     fwrite(ids, 4, B, out);
     fwrite(st, 4, B, out);
-    free(x); free(prm); free(u); free(ids); free(st); free(stats);
+    free(x); free(prm); free(u); free(c); free(ids); free(st); free(stats);
     fprintf(stderr, "group V=%d B=%d done\n", V, B);
   }
   fclose(out);

@@ -65,9 +65,34 @@ inline uint64_t xchg(uint64_t v, F f, const char* file = __builtin_FILE(),
 template <class T> inline uint64_t bits(T v) { uint64_t b = 0; std::memcpy(&b, &v, sizeof(T)); return b; }
 template <class T> inline T from(uint64_t b) { T v; std::memcpy(&v, &b, sizeof(T)); return v; }
 }  // namespace emu
+namespace emu {
+// With EMU_CHECK_BARRIERS set: every work-item of a workgroup must reach the
+// same __syncthreads (on the GPU, waves at different ones go on together,
+// a barrier out of step).  The driver ends each work-item with one more
+// (leave), so one that returns early is found too.
+struct BlockSite { const char* file; int line; };
+inline BlockSite block_site[1024];
+inline void block_wait(const char* file, int line) {
+  static const bool on = std::getenv("EMU_CHECK_BARRIERS") != nullptr;
+  at(file, line);
+  if (!on) {
+    block_bar->arrive_and_wait();
+    return;
+  }
+  block_site[threadIdx.x] = {file, line};
+  block_bar->arrive_and_wait();
+  const BlockSite s0 = block_site[0];
+  const bool same = s0.line == line && std::strcmp(s0.file, file) == 0;
+  block_bar->arrive_and_wait();
+  if (same) return;
+  std::fprintf(stderr, "work-item %u at barrier %s:%d, work-item 0 at %s:%d\n", threadIdx.x, file,
+               line, s0.file, s0.line);
+  std::_Exit(6);
+}
+inline void leave() { block_wait("(returned)", 0); }
+}  // namespace emu
 inline void __syncthreads(const char* file = __builtin_FILE(), int line = __builtin_LINE()) {
-  emu::at(file, line);
-  emu::block_bar->arrive_and_wait();
+  emu::block_wait(file, line);
 }
 inline void __threadfence() { std::atomic_thread_fence(std::memory_order_seq_cst); }
 inline void __threadfence_block() { std::atomic_thread_fence(std::memory_order_seq_cst); }

@@ -7,7 +7,9 @@ allocation, so an out-of-bounds access fails the run.  On top-p / min-p rows
 with deep nuclei (fp32 rows of odd length, so most rows start unaligned, and
 bf16 rows full of ties) every row a path decides must sample the oracle's
 id; a row it hands back (-2) is allowed only where the test expects it.
-CPU only."""
+Typical-p rows are run with the entropy shift the chunk sums give, every
+barrier of theirs checked to be the same one for all work-items.  CPU
+only."""
 from __future__ import annotations
 
 import os
@@ -97,21 +99,25 @@ def _splits_a_tie(row: np.ndarray, prm: RowParams) -> bool:
     return int(np.sum(p[order[:cut]] == v)) < int(np.sum(p == v))
 
 
-def _run(groups, mode: int = 0):
+def _run(groups, mode: int = 0, env=None):
+    """groups: (kind, logits, params, rows handed back, uniforms or None[,
+    the typical rows' entropy shifts, NaN: the row's own])."""
     us = []
     with tempfile.TemporaryDirectory() as tmp:
         exe = _build(tmp)
         fin, fout = os.path.join(tmp, "in.bin"), os.path.join(tmp, "out.bin")
         with open(fin, "wb") as f:
             f.write(struct.pack("i", len(groups)))
-            for kind, x, prm, _, ug in groups:
+            for kind, x, prm, _, ug, *shift in groups:
                 B, V = x.shape
+                c = np.asarray(shift[0] if shift else [np.nan] * B)
                 u = ug if ug is not None else np.random.default_rng(B * 7 + V).random(B)
                 us.append(u)
                 f.write(struct.pack("iii", B, V, 1 if kind == "bf16" else 0))
-                for a in (x, pack_rows(prm), u.astype(np.float64)):
+                for a in (x, pack_rows(prm), u.astype(np.float64), c.astype(np.float64)):
                     f.write(np.ascontiguousarray(a).tobytes())
-        r = subprocess.run([exe, fin, fout, str(mode)], capture_output=True, text=True, timeout=900)
+        r = subprocess.run([exe, fin, fout, str(mode)], capture_output=True, text=True, timeout=900,
+                           env=dict(os.environ, **(env or {})))
         assert r.returncode == 0, r.stderr[-4000:]
         out = open(fout, "rb").read()
     return _check(groups, us, out)
@@ -120,7 +126,7 @@ def _run(groups, mode: int = 0):
 def _check(groups, us, out) -> int:
     off = 0
     decided = 0
-    for (kind, x, prm, back, _), u in zip(groups, us):
+    for (kind, x, prm, back, *_), u in zip(groups, us):
         B, V = x.shape
         ids = np.frombuffer(out, np.int32, B, off)
         off += 8 * B
@@ -214,3 +220,49 @@ def test_counted_deep_path_kept_range_through_zero():
     tiny = np.abs(rows) < 2.0 ** -20
     assert tiny[:3].sum(axis=1).min() >= 60 and tiny[3].all()
     assert _run([("bf16", xb, prm, set(), None)], 16) == 4
+
+
+def _cut_within(row: np.ndarray, member: np.ndarray, temperature: float) -> float:
+    """A typical_p whose cut keeps about half of a group of equal
+    typical-order distances (``member``: one of its ids)."""
+    with np.errstate(all="ignore"):
+        P = R.tempered_probs(row.astype(np.float64), temperature)
+    logp = np.log(np.maximum(P, 1e-38))
+    dist = np.abs(logp - (P * logp).sum())
+    order = np.argsort(dist, kind="stable")
+    run = np.cumsum(P[order])
+    pos = np.flatnonzero(dist[order] == dist[member])
+    assert pos.size > 8
+    j = pos[pos.size // 2]
+    return float((run[j - 1] + run[j]) / 2)
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_typical_cut_in_a_group_of_equal_distances(kind):
+    """Typical-p rows whose cut splits a group of equal distances: zeros of
+    both signs and, in fp32, values so small that x - M is the same for all
+    of them, are one value (the survivors spread over the ids); the order's
+    two sides at the very same distance are handed back, by every work-item
+    at the same barrier."""
+    rng = np.random.default_rng(41)
+    V = 12000
+    x = (np.round(rng.normal(0, 2.0, (4, V)) * 8) / 8).astype(np.float32)
+    prm = []
+    for b in range(3):
+        zero = np.flatnonzero(x[b] == 0.0)
+        x[b, zero[rng.random(zero.size) < 0.5]] = np.float32(-0.0)
+        if b == 1:
+            x[b, zero] = rng.choice([1e-30, -3e-25, 0.0, -0.0, 2e-20], zero.size).astype(np.float32)
+        T = (1.0, 1.0, 0.7)[b]
+        p = _cut_within(x[b], int(zero[0]), T)
+        assert 0.02 < p < 1.0
+        prm.append(RowParams(temperature=T, typical_p=p))
+    # d = -0.5 and -1.5 around c = 1: the same distance on both sides
+    x[3] = np.repeat(np.float32([0.0, -0.5, -1.0, -1.5, -6.0]), (1, 300, 400, 300, V - 1001))
+    P = np.exp(x[3].astype(np.float64))
+    P /= P.sum()
+    prm.append(RowParams(temperature=1.0, typical_p=float(P[x[3] == -1.0].sum() +
+                                                          40.5 * P[x[3] == -0.5][0])))
+    c = np.array([np.nan] * 3 + [1.0])
+    xs = f32_to_bf16_rne(x) if kind == "bf16" else x
+    assert _run([(kind, xs, prm, {3}, None, c)], env={"EMU_CHECK_BARRIERS": "1"}) == 3
