@@ -305,6 +305,9 @@ __global__ __launch_bounds__(HEAD_WG) void head_merge(HeadArgs A) {
   }
 }
 
+constexpr int HEAD_VT_MIN = 64;              // the smallest vocab tile of a plan
+static int vocab_tiles(int V, int vt) { return (int)(((int64_t)V + vt - 1) / vt); }
+
 // The launch of a batch of B rows over V vocab rows: batch tiles of 32, 64,
 // 128 or 256 rows, and workgroups of 64 (4 waves), 128 or 256 vocab rows (8
 // waves of 16 or 32).
@@ -320,7 +323,7 @@ static HeadPlan head_plan(int B, int V) {
   if (p.nt == 0) {
     // small workgroups balance best at every V: 120 against 134 us for 128
     // vocab rows at V = 80000, 11 against 15 us at V = 4080
-    p.vt = 64;
+    p.vt = HEAD_VT_MIN;
   } else if (p.nt < 3) {
     // 128 vocab rows (B = 64: 57 against 62 us at V = 32000) once they fill
     // most of the CUs; below, 64 (18 against 24 us at V = 16000)
@@ -342,7 +345,7 @@ static HeadPlan head_plan(int B, int V) {
 int launch_head(const HeadArgs& A0, hipStream_t s) {
   HeadArgs A = A0;
   const HeadPlan p = head_plan(A.B, A.V);
-  A.nvt = (A.V + p.vt - 1) / p.vt;
+  A.nvt = vocab_tiles(A.V, p.vt);
   // weight rows a multiple of 4096 bytes apart: four starting points in k
   // (each quarter a whole number of ring turns)
   const bool seg = A.ldw % 2048 == 0 && A.D % (4 * WIDE_RING * WIDE_SK) == 0;
@@ -369,10 +372,13 @@ int launch_head(const HeadArgs& A0, hipStream_t s) {
 
 extern "C" {
 
+// The keys of the smallest vocab tile any plan takes: the size grows with B
+// and with V, though the plan's own tile does not, so a workspace of the
+// largest call serves every smaller one (B = 256, V = 128256: 4.1 MB, of
+// which that plan writes 1.0).
 size_t cx_lmhead_workspace_bytes(int32_t B, int32_t V) {
   if (B <= 0 || V <= 0) return 256;
-  const int vt = cx::head_plan(B, V).vt;
-  return ((size_t)B * ((V + vt - 1) / vt) * 8 + 255) & ~(size_t)255;
+  return ((size_t)B * cx::vocab_tiles(V, cx::HEAD_VT_MIN) * 8 + 255) & ~(size_t)255;
 }
 
 int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* weight,
@@ -388,9 +394,9 @@ int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* w
     return cx::api_fail(CX_EINVAL, "null pointer argument");
   if ((((uintptr_t)hidden | (uintptr_t)weight) & 15) || ((ldh | ldw) & 7))
     return cx::api_fail(CX_EINVAL, "hidden and weight rows must be 16-byte aligned");
-  if (ws_bytes < cx_lmhead_workspace_bytes(B, V))
-    return cx::api_fail(CX_ENOSPACE, "workspace holds %zu bytes, needs %zu", ws_bytes,
-                        cx_lmhead_workspace_bytes(B, V));
+  const size_t need = (size_t)B * cx::vocab_tiles(V, cx::head_plan(B, V).vt) * 8;
+  if (ws_bytes < need)
+    return cx::api_fail(CX_ENOSPACE, "workspace holds %zu bytes, needs %zu", ws_bytes, need);
   cx::HeadArgs A;
   A.hidden = hidden; A.weight = weight; A.ldh = ldh; A.ldw = ldw;
   A.B = B; A.D = D; A.V = V;

@@ -225,7 +225,8 @@ int cx_spec_verify_host(const float* target, const float* draft, const int32_t* 
  *  out_logits nullable [B, V] fp32: every logit (verification only; this
  *             write is what the fusion saves)
  *  workspace  device scratch of cx_lmhead_workspace_bytes(B, V) bytes; any
- *             contents.
+ *             contents.  The size grows with B and with V: one workspace of
+ *             the largest batch and vocabulary serves every smaller call.
  * Device pointers, stream-ordered, no synchronisation, no allocation.
  */
 int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* weight,

@@ -45,6 +45,17 @@ def test_workspace_sizes_are_host_only():
     assert lib.cx_spec_verify_workspace_bytes(32, 8, 128256) > 0
 
 
+def test_lmhead_workspace_grows_with_batch_and_vocabulary():
+    """One workspace of the largest call serves every smaller one, across the
+    edges where the kernel's batch and vocab tiles change."""
+    lib = _lib.load()
+    Bs = [1, 2, 16, 31, 32, 33, 40, 64, 65, 127, 128, 129, 200, 255, 256, 257, 320, 512, 513]
+    Vs = [1, 63, 64, 65, 777, 4099, 16000, 16384, 16385, 16400, 20479, 20480, 20481, 32000, 32768,
+          32769, 40001, 50257, 65537, 128256, 256000]
+    size = np.array([[lib.cx_lmhead_workspace_bytes(b, v) for v in Vs] for b in Bs])
+    assert (np.diff(size, axis=0) >= 0).all() and (np.diff(size, axis=1) >= 0).all()
+
+
 def test_bad_arguments_fail_before_any_device_work():
     lib = _lib.load()
     x = np.zeros((2, 8), np.float32)
