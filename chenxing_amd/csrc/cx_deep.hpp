@@ -49,8 +49,7 @@
 // where used, so the loads stay in flight; bf16 rows at odd addresses load
 // value by value.
 //
-// The sums that decide run in a fixed order in fp64 (but the kept gathered
-// terms, added as integers in units of 2^-51).  Each term is within 1 ulp
+// The sums that decide run in a fixed order in fp64.  Each term is within 1 ulp
 // (2.5 ulp for the table product), fp64 sums of at most 2^20 terms within
 // 2^20 ulp, and the reference's own cumulative sums within 4e-11 (relative)
 // of exact: a decision closer to its threshold than 5e-11 of the total
@@ -447,7 +446,6 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   __shared__ double tab[64];
   __shared__ double s_d[2 * NWAVE + 4];
   __shared__ double s_wm[NWAVE];                     // kept mass per wave range / sixteenth
-  __shared__ unsigned long long s_kept[NWAVE];       // per range: the gathered kept terms
   __shared__ int s_i[4];
   __shared__ int s_g[2];
   const int t = threadIdx.x, l = lane_id(), w = wave_id();
@@ -502,13 +500,13 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     return wbits - 1 - (int)__builtin_ceilf(top * LOG2E);
   };
   const bool cut = TYP || P.top_p < 1.0;
-  // (a typical target so small that 2^-51 units no longer resolve it)
+  // (below, the decision margin, relative to the whole row's sum, is wide
+  // beside the kept mass: the multi-pass path)
   if (TYP && !(P.typical_p >= 0.02)) return false;
   // (bf16 rows at odd addresses have the term-table pass only)
   if (!VEC && !use_tab) return false;
   for (int b = t; b < 2 * DNB; b += WG) h[b] = 0u;
   for (int b = t; b < NWAVE * NWAVE; b += WG) ab[b] = 0.0;
-  if (t < NWAVE) s_kept[t] = 0ull;
   if (t == 0) { s_i[0] = 0; s_i[2] = 0; }
   load_exp64_tab(tab);                               // its barrier also orders the clears
 
@@ -615,6 +613,7 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   float xcut = -__builtin_inff();
   double dcut = 0.0;                                 // TYP: the cut distance
   int g0 = 0, gn = 0, gj = 0;                        // the cut value's group: none
+  double kept = 0.0;                                 // range w's kept gathered terms, lane l's part
   if (cut) {
     const double tgt = (TYP ? P.typical_p : P.top_p) * S;
     const double total = lane_read(block_sum(t < NWAVE * NWAVE ? ab[t] : 0.0, s_d), 0);
@@ -720,15 +719,20 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     g0 = __builtin_amdgcn_readfirstlane(s_g[0]);
     gn = __builtin_amdgcn_readfirstlane(s_g[1]) - g0;
     gj = js + 1 - g0;
-    // the kept part of the gathered elements, per range: the entries above
-    // the cut value and the group's survivors
+    // the kept part of the gathered elements, the entries above the cut value
+    // and the group's survivors, in the keys' place (done with); wave w sums
+    // range w's in their order
+    if (P.min_p <= 0.0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 4 * t + j;
-      if (e < g0 || (e < g0 + gn && spread_keeps(e - g0, gj, gn, V <= TIE_NET)))
-        atomicAdd(s_kept + gi[e] / L, (unsigned long long)(qv[j] * 2251799813685248.0));
+      for (int j = 0; j < 4; ++j) {
+        const int e = 4 * t + j;
+        const bool k = e < g0 || (e < g0 + gn && spread_keeps(e - g0, gj, gn, V <= TIE_NET));
+        if (e < ng) gk[e] = (uint64_t)__double_as_longlong(k ? qv[j] : 0.0);
+      }
+      __syncthreads();
+      for (int e = l; e < g0 + gn; e += 64)
+        kept += (uint32_t)(gi[e] - w * L) < (uint32_t)L ? __longlong_as_double((long long)gk[e]) : 0.0;
     }
-    __syncthreads();
   }
 
   // kept: above the cut value, or in its group among the survivors (the
@@ -781,9 +785,9 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   // ---- each range's kept mass: its sums above the cut's buckets and its
   // kept gathered terms (no min-p), or pass 3
   if (minp <= 0.0) {
-    double m = l < NWAVE ? ab[w * NWAVE + l] : 0.0;
+    double m = (l < NWAVE ? ab[w * NWAVE + l] : 0.0) + kept;
     m = wave_reduce(m, OpAdd());
-    if (l == 0) s_wm[w] = m + (double)s_kept[w] * 4.440892098500626e-16;   // 2^-51
+    if (l == 0) s_wm[w] = m;
     __syncthreads();
   } else {
     const double m = wave_mass(w * L, w * L + L);

@@ -266,3 +266,32 @@ def test_typical_cut_in_a_group_of_equal_distances(kind):
     c = np.array([np.nan] * 3 + [1.0])
     xs = f32_to_bf16_rne(x) if kind == "bf16" else x
     assert _run([(kind, xs, prm, {3}, None, c)], env={"EMU_CHECK_BARRIERS": "1"}) == 3
+
+
+def test_typical_kept_terms_summed_in_full():
+    """A typical-p row whose kept terms are all gathered and lie just below
+    multiples of 2^-51, their sum 0.02 of the row's: its draw lies 1e-11 of
+    the kept mass from a step, so it is handed back; sums in integers of
+    2^-51 would put it 7e-11 to the wrong side."""
+    rng = np.random.default_rng(43)
+    V, n, c = 5000, 4090, 12.2
+    w = 40.0 / 4096                                        # one bucket of distances
+    lo, hi = np.float32(5 * w - c + 1e-5), np.float32(6 * w - c - 1e-5)
+    cand = np.arange(hi.view(np.uint32), lo.view(np.uint32), dtype=np.uint32).view(np.float32)
+    frac = np.modf(np.exp(cand.astype(np.float64)) * 2.0 ** 51)[0]
+    vals = cand[np.argsort(-frac)[:n]]
+    x = np.full((1, V), -30.0, np.float32)
+    x[0, :n] = vals[rng.permutation(n)]
+    x[0, V - 1] = 0.0
+    q = np.exp(x[0].astype(np.float64))
+    order = np.argsort(np.abs(x[0].astype(np.float64) + c), kind="stable")
+    run = np.cumsum(q[order])
+    j = n - 60
+    p = float((run[j - 1] + run[j]) / 2 / q.sum())
+    assert 0.02 < p < 0.03
+    kept = np.sort(order[:j + 1])
+    cum = np.cumsum(q[kept])
+    k = kept.size - 40
+    u = np.array([(cum[k] + 1e-11 * cum[-1]) / cum[-1]])
+    prm = [RowParams(temperature=1.0, typical_p=p)]
+    assert _run([("f32", x, prm, {0}, u, np.array([c]))]) == 0
