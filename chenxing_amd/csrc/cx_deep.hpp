@@ -8,7 +8,7 @@
 //
 //   pass 1  where the cut lies: a histogram of the terms exp((x - M) / T) (M
 //           the row maximum) over DNB value buckets linear in (M - x) / T on
-//           [0, DSPAN), the terms in fp32 rounded to integers of 12 bits or
+//           [0, DSPAN), the terms in fp32 rounded to integers of 11 bits or
 //           more in a scale of their bucket, and from it the buckets the
 //           running sum can reach top_p in, the roundings allowed for:
 //           usually one
@@ -487,12 +487,15 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     const double v = dist(x) * (double)DSCALE;
     return v < (double)DNB ? (int)v : -1;
   };
-  // pass 1's integers have wbits bits, as many as keep V of them below 2^32:
-  // 2^s brings the bucket's largest term (of the typical order's upper side,
-  // d + c > 0, where the terms grow with the distance) just below 2^wbits.
-  // A bucket's sum is then within 2^-wbits of its terms' (fp32 terms: 1e-5).
+  // pass 1's integers: 2^s brings the bucket's largest term (of the typical
+  // order's upper side, d + c > 0, where the terms grow with the distance)
+  // into (2^(wbits - 2), 2^(wbits - 1)], so V of them, the fp32 error
+  // included, stay below 2^32.  Rounding one of them to an integer changes it
+  // by at most 1.02 * 2^(1 - wbits) of itself (a bucket's smallest is 0.99 of
+  // its largest), the fp32 term by 2e-5: eps bounds the relative error of any
+  // sum of them.
   const int wbits = __clz(V);
-  const double eps = __builtin_ldexp(1.0, -wbits) + 1e-5;
+  const double eps = 1.02 * __builtin_ldexp(2.0, -wbits) + 2e-5;
   constexpr float LOG2E = 1.44269504f;
   const float cf = (float)c;
   auto weight_scale = [&](int b, bool up) -> int {
@@ -539,17 +542,26 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
     const double Sa = block_sum(c4, s_d);
     const double p = TYP ? P.typical_p : P.top_p;
     double incl = block_excl_scan_d(c4, s_d);
+    // The mass up to a bucket's end against the mass past it, a : r, each
+    // within eps: blo is the first bucket that can reach p, bhi the first
+    // that must.  (Against the whole row's sum, top_p within eps of 1 would
+    // have no upper bucket.)  slack: the mass below the span, at most
+    // V exp(-40), and the rounding of r.
+    const double slack = 5e-12 * Sa;
     int b0 = INT_MAX, b1 = INT_MAX;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       incl += vb[j];
-      if (b0 == INT_MAX && vb[j] != 0.0 && incl >= (p - eps) * Sa) b0 = 4 * t + j;
-      if (b1 == INT_MAX && vb[j] != 0.0 && incl >= (p + eps) * Sa) b1 = 4 * t + j;
+      const double a = incl * (1.0 - p), r = (Sa - incl) * p;
+      if (b0 == INT_MAX && vb[j] != 0.0 && a * (1.0 + eps) >= r * (1.0 - eps) - slack)
+        b0 = 4 * t + j;
+      if (b1 == INT_MAX && vb[j] != 0.0 && a * (1.0 - eps) >= r * (1.0 + eps) + slack * p)
+        b1 = 4 * t + j;
     }
     // (uniform values, here and below, into scalar registers)
     blo = __builtin_amdgcn_readfirstlane(block_min(b0, red_i, INT_MAX));
-    bhi = __builtin_amdgcn_readfirstlane(min(block_min(b1, red_i, INT_MAX), DNB - 1));
-    if (blo == INT_MAX) return false;                // NaN sums
+    bhi = __builtin_amdgcn_readfirstlane(block_min(b1, red_i, INT_MAX));
+    if (bhi == INT_MAX) return false;                // NaN sums, or p within 6e-12 of 1
   }
   if (use_tab) {
     deep_build_tables(ta, tb, tc, M, invT, tab);

@@ -295,3 +295,18 @@ def test_typical_kept_terms_summed_in_full():
     u = np.array([(cum[k] + 1e-11 * cum[-1]) / cum[-1]])
     prm = [RowParams(temperature=1.0, typical_p=p)]
     assert _run([("f32", x, prm, {0}, u, np.array([c]))]) == 0
+
+
+def test_cuts_near_the_whole_mass():
+    """top_p and typical_p so near 1 that the mass past the cut is below pass
+    1's error on the whole row's: the cut is bracketed by the mass past it
+    too, so the long tail behind it does not overflow the gather."""
+    rng = np.random.default_rng(47)
+    V = 30011
+    x = rng.normal(0, 1.0, (4, V)).astype(np.float32)
+    for b in range(4):
+        x[b, rng.choice(V, 12000, replace=False)] -= np.float32(16.0)
+    prm = [RowParams(temperature=1.0, top_p=0.99999), RowParams(temperature=1.0, top_p=0.999995),
+           RowParams(temperature=0.9, top_p=0.99995, min_p=1e-6),
+           RowParams(temperature=1.0, typical_p=0.99999)]
+    assert _run([("f32", x, prm, set(), None)]) == 4
