@@ -97,24 +97,25 @@ __global__ __launch_bounds__(WG) void slow_kernel(SampleArgs A) {
     state = r == FIN_REFINE ? REFINE : r == FIN_WHOLE ? WHOLE : MULTIPASS;
     __syncthreads();
   }
-  // the long paths from here on: with their registers (the arguments above
-  // all) out of the finisher's way, 64 top-p rows of 128256 take 39.65
-  // instead of 39.84 us a call
-  const SampleArgs& D = args_again();
   if (state == WHOLE) {
-    const cx_row_params P = D.prm[row];
+    const cx_row_params P = A.prm[row];
     WholeSums Z;
-    const int r = whole_finish(D, row, P, red_d, red_i, Z);
+    const int r = whole_finish(A, row, P, red_d, red_i, Z);
     if (r == WHOLE_DONE) return;
     __syncthreads();
-    if (r == WHOLE_TYP && deep_row(D, row, dyn, red_d, red_i, &Z)) return;
+    if (r == WHOLE_TYP && deep_row(A, row, dyn, red_d, red_i, &Z)) return;
   } else {
-    if (state == REFINE && refine_row(D, row, dyn, red_d, red_i)) return;
+    if (state == REFINE && refine_row(A, row, dyn, red_d, red_i)) return;
     __syncthreads();
-    if (deep_row(D, row, dyn, red_d, red_i)) return;
+    if (deep_row(A, row, dyn, red_d, red_i)) return;
   }
   __syncthreads();
-  slow_row(D, row, dyn, red_d, red_i);
+  // (the arguments above, live across the finisher, spill into vector lanes
+  // on its critical path: 64 top-p rows of 128256 40.4 -> 39.8 us a call.
+  // The deep paths on the second copy too, and this path's row scalars in
+  // scalar registers, cost the multi-pass path 28 %: 8 penalised rows of
+  // 2000 140 -> 179 us.)
+  slow_row(args_again(), row, dyn, red_d, red_i);
 }
 
 // finish16_kernel's work items, in the order they are taken: 1 for a row

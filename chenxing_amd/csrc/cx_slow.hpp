@@ -597,8 +597,8 @@ __device__ inline void slow_row(const SampleArgs& A, int row, unsigned char* dyn
   }
   block_argmax(bv, bi, red_d, red_i);
   ni = block_min(ni, red_i, INT_MAX);
-  mx = lane_read(bv, 0);                             // uniform: into scalar registers
-  mn = lane_read(block_min(mn, red_d, __builtin_inf()), 0);
+  mx = bv;
+  mn = block_min(mn, red_d, __builtin_inf());
   const int amax = ni != INT_MAX ? ni : (bi == INT_MAX ? 0 : bi);
   if (P.temperature == 0.0) {                                // sampler.py:114-115
     if (A.out_probs) {
@@ -611,7 +611,7 @@ __device__ inline void slow_row(const SampleArgs& A, int row, unsigned char* dyn
     }
     return;
   }
-  const double invT = lane_read(1.0 / P.temperature, 0);
+  const double invT = 1.0 / P.temperature;
   bool degenerate = ni != INT_MAX || mx == __builtin_inf() || mx == -__builtin_inf();
   R.M = mx;
   R.invT = invT;
@@ -625,7 +625,7 @@ __device__ inline void slow_row(const SampleArgs& A, int row, unsigned char* dyn
       s += exp((v - mx) * invT);
       if (under) s1 += exp(v - mx);
     }
-    R.S = lane_read(block_sum(s, red_d), 0);
+    R.S = block_sum(s, red_d);
     if (under) {
       double S1 = block_sum(s1, red_d);
       if (pow(1.0 / S1, invT) == 0.0) degenerate = true;
