@@ -467,8 +467,10 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   double* ta = (double*)(dyn + DEEP_OFF_X);
   double* tb = ta + 4096;
   double* tc = tb + 2048;
-  // the term tables: bf16 rows whose |x| / T stays below 7000
-  const bool use_tab = R.bf16 && (fabs(M) + 40.0 * P.temperature) * invT < 7000.0;
+  // the term tables: bf16 rows of whole dwords whose |x| / T stays below
+  // 7000 (others take the exponential itself: one pass for both is enough
+  // where every load is a single value)
+  const bool use_tab = VEC && R.bf16 && (fabs(M) + 40.0 * P.temperature) * invT < 7000.0;
   const int cap = R.bf16 ? DCAP16 : DCAP;
   unsigned char* gbase = R.bf16 ? dyn : dyn + DEEP_OFF_X;
   uint64_t* gk = (uint64_t*)gbase;
@@ -506,8 +508,6 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   // (below, the decision margin, relative to the whole row's sum, is wide
   // beside the kept mass: the multi-pass path)
   if (TYP && !(P.typical_p >= 0.02)) return false;
-  // (bf16 rows at odd addresses have the term-table pass only)
-  if (!VEC && !use_tab) return false;
   for (int b = t; b < 2 * DNB; b += WG) h[b] = 0u;
   for (int b = t; b < NWAVE * NWAVE; b += WG) ab[b] = 0.0;
   if (t == 0) { s_i[0] = 0; s_i[2] = 0; }
@@ -616,8 +616,8 @@ __device__ __forceinline__ bool deep_row_impl(const SampleArgs& A, int row, cons
   };
   // (a branch per element would leave each wave waiting for its own table
   // read: 51 us at V = 128256 fp32)
-  if (use_tab) pass2(DeepFlag<true>());
-  else if constexpr (VEC) pass2(DeepFlag<false>());
+  if (use_tab) pass2(DeepFlag<VEC>());
+  else pass2(DeepFlag<false>());
   const double S = lane_read(block_sum(s, s_d), 0);
   if (block_max(bad, red_i, 0)) return false;        // NaN (or a value above M)
   const double tolS = DTOL * S;

@@ -310,3 +310,17 @@ def test_cuts_near_the_whole_mass():
            RowParams(temperature=0.9, top_p=0.99995, min_p=1e-6),
            RowParams(temperature=1.0, typical_p=0.99999)]
     assert _run([("f32", x, prm, set(), None)]) == 4
+
+
+def test_bf16_rows_at_odd_addresses():
+    """bf16 rows an odd number of elements apart (read value by value),
+    whose logits over T are small enough for the term tables and too large:
+    the same passes."""
+    rng = np.random.default_rng(53)
+    V = 20011
+    x = rng.normal(0, 2.0, (4, V)).astype(np.float32)
+    x[2:] = np.float32(-8192.0) + np.float32(32.0) * np.floor(rng.exponential(1.5, (2, V)))
+    xb = f32_to_bf16_rne(np.where(x < -8500, np.float32(-8500.0), x).astype(np.float32))
+    prm = [RowParams(temperature=1.5, top_p=0.9), RowParams(temperature=1.2, top_p=0.6, min_p=1e-4),
+           RowParams(temperature=1.0, top_p=0.9), RowParams(temperature=0.9, top_p=1.0, min_p=1e-9)]
+    assert _run([("bf16", xb, prm, set(), None)]) == 4
