@@ -179,12 +179,7 @@ static int sample_impl(const void* logits, int dtype, int64_t ld, int32_t B, int
   A.all_slow = dtype == 2;
   A.logV = log((double)V);
   const int esz = dtype == 2 ? 8 : (dtype == 1 ? 2 : 4);
-  // 16-byte buffer loads take any dword address, and their range check is
-  // per dword: every fp32 row, and bf16 rows an even number of elements
-  // apart, are read as vectors (37 rows of 50257 fp32, mixed filters: 131 to
-  // 88 us in slow_kernel, 34 to 20 us in the fused kernel against element
-  // loads).
-  A.vec_ok = (((uintptr_t)logits) % 4 == 0) && ((ld * esz) % 4 == 0);
+  A.vec_ok = vec_flags(logits, ld * esz, A.split_len);
   slow_layout(A, V, ldh);
   fused_layout(A, ldh);
   if (A.lds_bytes > FUSED_LDS_MAX)

@@ -299,7 +299,7 @@ __device__ __forceinline__ WholeSlice whole_slice_of(const SampleArgs& A, int sp
   const int ne = A.bf16 ? 8 : 4;
   w.lo = split * A.split_len;
   w.hi = min(A.V, w.lo + A.split_len);
-  w.s0 = A.vec_ok && w.hi > w.lo ? w.lo + (w.hi - w.lo) / ne * ne : w.lo;
+  w.s0 = (A.vec_ok & VEC_STREAM) && w.hi > w.lo ? w.lo + (w.hi - w.lo) / ne * ne : w.lo;
   w.nvc = (w.s0 - w.lo + WCH - 1) / WCH;
   w.nsc = w.hi > w.s0 ? (w.hi - w.s0 + WCH - 1) / WCH : 0;
   return w;

@@ -91,7 +91,7 @@ struct SampleArgs {
   Cand* cands;            // [B * nsplit * CAPS]
   int32_t nsplit, split_len;
   int32_t ns, ns_log2;    // penalty hash slots (power of two, >= 2 x window) and log2
-  int32_t vec_ok;         // rows start at whole dwords (16-byte buffer loads need no more)
+  int32_t vec_ok;         // VEC_LOADS, VEC_STREAM (vec_flags)
   int32_t off_bitmap, off_hword, off_hval, off_dense, off_wkey, off_widx, off_gather;
   int32_t lds_bytes;      // fused kernel dynamic LDS
   int32_t bf16;           // logits are bf16 bit patterns
@@ -179,6 +179,29 @@ struct SampleWorkspace {
 };
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
+
+// SampleArgs::vec_ok.  16-byte buffer loads take any dword address, and their
+// range check is per dword: every fp32 row, and bf16 rows an even number of
+// elements apart, can be read as vectors (VEC_LOADS).
+constexpr int VEC_LOADS = 1;
+// VEC_STREAM: the fused kernel streams them so, too: 16-byte aligned rows, and
+// the others in slices of at least VEC_MIN elements.  A shorter slice is only a
+// few chunks of 1024 elements, each one wave's: the waves without one stand
+// idle, and the candidates land in a few waves' buffers, which overflow, where
+// element loads spread both over all 16.  (4 fp32 top-p rows, vectors against
+// elements: V = 257 25 and 21 us, 1001 39 and 22, 3001 54 and 27, 6001 58 and
+// 49, 9001 62 and 64, 16001 55 and 73.)  Top-k rows of one chunk whose k the
+// one-wave finish takes are better off in one wave's buffer (VEC_TOPK; 4 rows
+// of 257: 15 against 62 us, of 3001 89 against 82; with penalties too, 4 bf16
+// rows of 1002 27 against 126 us, 4 fp32 rows of 257 101 against 98).
+constexpr int VEC_STREAM = 2;
+constexpr int VEC_MIN = 8192;
+constexpr int VEC_TOPK = 64;
+inline int vec_flags(const void* logits, int64_t row_bytes, int split_len) {
+  if ((uintptr_t)logits % 4 != 0 || row_bytes % 4 != 0) return 0;
+  const bool aligned = (uintptr_t)logits % 16 == 0 && row_bytes % 16 == 0;
+  return aligned || split_len >= VEC_MIN ? VEC_LOADS | VEC_STREAM : VEC_LOADS;
+}
 
 constexpr int SLICE_MAX = 1 << 18;        // elements per slice (bitmap index limit)
 constexpr int SLICE_CAP = 8;              // slices per row (V < 2^20 needs at most 4)

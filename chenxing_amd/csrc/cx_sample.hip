@@ -1181,8 +1181,7 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
 #pragma unroll
   for (int k = 0; k < HPT; ++k)
     hid[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(hrs, (t + k * WG) * 4, 0, 0);
-  const int nv = A.vec_ok ? (hi - lo) / NE : 0;       // whole vectors of the slice
-  const int s0 = lo + nv * NE;                         // first scalar element
+  int nv = A.vec_ok ? (hi - lo) / NE : 0;             // whole vectors of the slice
   const __amdgpu_buffer_rsrc_t rs = row_rsrc(rowp + (size_t)lo * (BF16 ? 2 : 4), nv * 16);
   const int ch0 = __builtin_amdgcn_readfirstlane(wave_id());
   typename E::V q[U], qn[U];
@@ -1210,6 +1209,12 @@ __global__ __launch_bounds__(WG) void sample_kernel(SampleArgs A) {
   const bool pen_on = wlen > 0 && (P0.repetition_penalty != 1.0 || P0.presence_penalty != 0.0 ||
                                    P0.frequency_penalty != 0.0);
   const bool whole = !pen_on && whole_row(A, P0);
+  // short rows off 16-byte boundaries: element loads, but for small top-k
+  // rows of one chunk
+  if (!(A.vec_ok & VEC_STREAM) &&
+      !(P0.top_k > 0 && P0.top_k <= VEC_TOPK && hi - lo <= 64 * U * NE))
+    nv = 0;
+  const int s0 = lo + nv * NE;                         // first scalar element
   if (pen_on && wlen > WIN_MAX) {                    // window longer than the LDS index
     if (t == 0) {
       my->flags = SF_UNSUPPORTED; my->ncand = 0; my->tau = 1u;

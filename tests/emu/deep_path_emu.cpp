@@ -78,7 +78,7 @@ int main(int argc, char** argv) {
     A.logits = x; A.ld = V; A.B = B; A.V = V; A.ldh = 0;
     A.prm = prm; A.u = u; A.out_id = ids; A.row_status = st; A.out_probs = nullptr;
     A.nsplit = 1; A.stats = stats; A.bf16 = bf16; A.logV = log((double)V);
-    A.vec_ok = ((uintptr_t)x % 4 == 0) && ((size_t)V * esz % 4 == 0);     // as the library sets it
+    A.vec_ok = vec_flags(x, (int64_t)V * esz, V);
     for (int row = 0; row < B; ++row) {
       unsigned char* dyn = (unsigned char*)malloc(lds);
       for (size_t i = 0; i < lds; ++i) dyn[i] = (unsigned char)(i * 131 + 7);

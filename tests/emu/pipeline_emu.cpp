@@ -199,7 +199,7 @@ int main(int argc, char** argv) {
     A.nsplit = nsplit;
     A.split_len = split_len_of(V, nsplit);
     A.logV = log((double)V);
-    A.vec_ok = ((uintptr_t)x) % 4 == 0;                     // as the library sets it
+    A.vec_ok = vec_flags(x, (int64_t)V * 4, A.split_len);
     slow_layout(A, V, H);
     fused_layout(A, H);
     for (unsigned blk = 0; blk < (unsigned)(B * nsplit); ++blk) {

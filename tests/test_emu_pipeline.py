@@ -218,6 +218,33 @@ def test_long_single_slice_rows_emulated():
         assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
 
 
+def test_short_rows_at_odd_addresses_emulated():
+    """Rows of two chunks and a bit off 16-byte boundaries: streamed element
+    by element, so every wave's buffer takes its share of the candidates and
+    the region decides flat top-p rows too (in vectors, three waves' buffers
+    would overflow)."""
+    V = 2001
+    rng = np.random.default_rng(59)
+    base = dict(temperature=2.0, top_k=0, top_p=0.9, min_p=0.0, typical_p=1.0,
+                repetition_penalty=1.0, n_keep=0)
+    rows = []
+    for i, (kw, hist) in enumerate([
+            (dict(), []), (dict(top_p=0.97), []), (dict(temperature=1.0), []),
+            (dict(top_k=40, temperature=0.8), [int(t) for t in rng.integers(0, V, 64)])]):
+        x = rng.normal(0.0, 2.0, V).astype(np.float32)
+        x[rng.choice(V, 5)] += 8.0
+        rows.append(cases.SamplerCase(f"short{i}", x, dict(base, **kw, seed=int(rng.integers(0, 2**31))),
+                                      hist))
+    with tempfile.TemporaryDirectory() as tmp:
+        (ids, st), = run_pipeline([rows], tmp)
+    for b, c in enumerate(rows):
+        u = np.random.default_rng(c.params["seed"]).random()
+        res = R.sample_row(c.logits, _params(c), c.hist, u, tie="spread")
+        assert int(st[b]) & 0xFF == res.status, (c.name, int(st[b]), res.status)
+        assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
+    assert all(int(st[b]) >> 8 == 0 for b in range(3)), st
+
+
 @pytest.mark.parametrize("V,nsplit", [(33000, None), (33001, None), (20003, "1")])
 def test_whole_rows_emulated(V, nsplit):
     """Rows drawn from whole (no filter, or typical-p alone): sliced with
