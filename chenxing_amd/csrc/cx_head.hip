@@ -8,8 +8,8 @@
 // MFMA (v_mfma_f32_16x16x32_bf16: A = 16 vocab rows x 32 k, B = 32 k x 16
 // batch rows, C = 16 x 16 fp32).  Two stream-ordered launches:
 //
-//   1. head_wide    one workgroup per (vocab tile, batch tile of up to 256
-//                   rows): the projection, reduced in registers and LDS to
+//   1. head_wide or  one workgroup per (vocab tile, batch tile of up to 256
+//      head_tall    rows): the projection, reduced in registers and LDS to
 //                   one 64-bit key per (vocab tile, batch row): the orderable
 //                   logit above the complement of the vocab id, so the
 //                   largest key is the largest logit with the lowest id on
@@ -19,6 +19,8 @@
 //
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <mutex>
 
 #include "cx_device.hpp"
 #include "cx_internal.hpp"
@@ -56,6 +58,44 @@ __device__ __forceinline__ u32x4 ld16(const uint16_t* p) {
 __device__ __forceinline__ uint64_t head_key(float x, int v) {
   const uint32_t k = x != x ? 0xFFFFFFFFu : f2key(x);
   return ((uint64_t)k << 32) | (uint32_t)~(uint32_t)v;
+}
+
+// A workgroup's keys: lane (g, c) of a wave holds the logits of vocab rows
+// v0 + 16 m + 4 g + j (j < 4) at batch rows b0 + 16 n + c.
+template <int NT, int MT, int NW>
+__device__ __forceinline__ void head_keys(const HeadArgs& A, const f32x4 (&acc)[MT][NT], int v0,
+                                          int b0, int vt, uint64_t (&s_key)[NW][16 * NT]) {
+  const int w = wave_id(), l = lane_id();
+  const int g = l >> 4, c = l & 15;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int b = b0 + 16 * n + c;
+    uint64_t key = 0;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int v = v0 + 16 * m + 4 * g + j;
+        const float x = acc[m][n][j];
+        if (v < A.V) {
+          const uint64_t k = head_key(x, v);
+          key = k > key ? k : key;
+          if (A.out_logits && b < A.B) A.out_logits[(size_t)b * A.V + v] = x;
+        }
+      }
+    uint64_t o = __shfl_xor(key, 16);
+    key = o > key ? o : key;
+    o = __shfl_xor(key, 32);
+    key = o > key ? o : key;
+    if (g == 0) s_key[w][16 * n + c] = key;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < 16 * NT && b0 + t < A.B; t += NW * 64) {
+    uint64_t key = s_key[0][t];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) key = s_key[k][t] > key ? s_key[k][t] : key;
+    A.part[(size_t)(b0 + t) * A.nvt + vt] = key;
+  }
 }
 
 // A wave owns 16 MT vocab rows and all the workgroup's 16 NT batch rows, so
@@ -243,35 +283,89 @@ __global__ __launch_bounds__(NW * 64, 1) void head_wide(HeadArgs A) {
         acc[0][m][n] = sum;
       }
   }
+  head_keys<NT, MT, NW>(A, acc[0], v0, b0, vt, s_key);
+}
+
+// Batches of up to 32 rows over a vocabulary whose tiles of 512 rows nearly
+// fill the CUs once (head_plan): one workgroup of 16 waves per tile, each
+// wave with 32 vocab rows.  The hidden states are staged in LDS a chunk of k
+// at a time (4736 k for 16 batch rows, 2304 for 32), so a wave runs its k loop
+// without barriers, its weights through a register ring of DEPTH blocks of
+// 128 k.  head_wide spends a barrier per 64 k and starts 2004 workgroups at
+// V = 128256, which shows where k is short or its walk starts at 0 everywhere:
+// B = 32, D = 512 36 against 31 us, D = 1536 85 against 75 us.
+constexpr int TALL_NW = 16, TALL_MT = 2;
+constexpr int TALL_VT = TALL_NW * TALL_MT * 16;
+constexpr int TALL_LDS = 152 * 1024;         // the staged chunk at most
+template <int NB>
+constexpr int tall_chunk() { return (TALL_LDS / (16 * NB * 2) - 8) / HEAD_KB * HEAD_KB; }
+
+template <int NB, int DEPTH>
+__global__ __launch_bounds__(TALL_NW * 64) void head_tall(HeadArgs A) {
+  extern __shared__ __align__(16) unsigned char head_lds[];
+  __shared__ uint64_t s_key[TALL_NW][16 * NB];
+  const int l = lane_id(), g = l >> 4, c = l & 15;
+  const int v0 = (int)blockIdx.x * TALL_VT + wave_id() * TALL_MT * 16;
+  const int KC = min(A.D, tall_chunk<NB>());
+  const int stride = KC + 8;                 // padded: the 16 rows of an operand in different banks
+  CX_LDS uint16_t* const hs = to_lds((uint16_t*)head_lds);
+  const CX_LDS uint16_t* const hl = hs + c * stride + 8 * g;
+  const uint16_t* wp[TALL_MT];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    const int b = b0 + 16 * n + c;
-    uint64_t key = 0;
+  for (int m = 0; m < TALL_MT; ++m)
+    wp[m] = A.weight + (size_t)min(v0 + 16 * m + c, A.V - 1) * A.ldw + 8 * g;
+  f32x4 acc[TALL_MT][NB];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < TALL_MT; ++m)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int v = v0 + 16 * m + 4 * g + j;
-        const float x = acc[0][m][n][j];
-        if (v < A.V) {
-          const uint64_t k = head_key(x, v);
-          key = k > key ? k : key;
-          if (A.out_logits && b < A.B) A.out_logits[(size_t)b * A.V + v] = x;
-        }
+    for (int n = 0; n < NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 ring[DEPTH][TALL_MT][4];
+  auto load = [&](u32x4 (&x)[TALL_MT][4], int k) {
+#pragma unroll
+    for (int m = 0; m < TALL_MT; ++m)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x[m][s] = ld16(wp[m] + k + 32 * s);
+  };
+  auto multiply = [&](const u32x4 (&x)[TALL_MT][4], int k) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      u32x4 h[NB];
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+        h[n] = *(const CX_LDS u32x4*)(hl + 16 * n * stride + k + 32 * s);
+#pragma unroll
+      for (int m = 0; m < TALL_MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, x[m][s]), __builtin_bit_cast(bf16x8, h[n]), acc[m][n],
+              0, 0, 0);
+    }
+  };
+  for (int k0 = 0; k0 < A.D; k0 += KC) {
+    const int kn = min(KC, A.D - k0);
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (d * HEAD_KB < kn) load(ring[d], k0 + d * HEAD_KB);
+    if (k0 > 0) __syncthreads();             // every wave is done with the last chunk
+    for (int i = threadIdx.x; i < 16 * NB * (kn / 8); i += TALL_NW * 64) {
+      const int r = i / (kn / 8), e = i % (kn / 8) * 8;
+      *(CX_LDS u32x4*)(hs + r * stride + e) =
+          *(const u32x4*)(A.hidden + (size_t)min(r, A.B - 1) * A.ldh + k0 + e);
+    }
+    __syncthreads();
+    for (int kb = 0; kb < kn; kb += DEPTH * HEAD_KB) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        const int k = kb + d * HEAD_KB;
+        if (k >= kn) break;
+        const int kx = k + (DEPTH - 1) * HEAD_KB;
+        if (kx < kn) load(ring[(d + DEPTH - 1) % DEPTH], k0 + kx);
+        multiply(ring[d], k);
       }
-    uint64_t o = __shfl_xor(key, 16);
-    key = o > key ? o : key;
-    o = __shfl_xor(key, 32);
-    key = o > key ? o : key;
-    if (g == 0) s_key[w][16 * n + c] = key;
+    }
   }
-  __syncthreads();
-  for (int t = threadIdx.x; t < ROWS && b0 + t < A.B; t += NW * 64) {
-    uint64_t key = s_key[0][t];
-#pragma unroll
-    for (int k = 1; k < NW; ++k) key = s_key[k][t] > key ? s_key[k][t] : key;
-    A.part[(size_t)(b0 + t) * A.nvt + vt] = key;
-  }
+  head_keys<NB, TALL_MT, TALL_NW>(A, acc, v0, 0, blockIdx.x, s_key);
 }
 
 // One workgroup per batch row: the largest key of its workgroups, four
@@ -310,20 +404,34 @@ static int vocab_tiles(int V, int vt) { return (int)(((int64_t)V + vt - 1) / vt)
 
 // The launch of a batch of B rows over V vocab rows: batch tiles of 32, 64,
 // 128 or 256 rows, and workgroups of 64 (4 waves), 128 or 256 vocab rows (8
-// waves of 16 or 32).
+// waves of 16 or 32), or of 512 (16 waves, head_tall).
 struct HeadPlan {
   int nt;            // index of the batch tile: 32 << nt rows
   int vt;            // vocab rows per workgroup
   int nby;           // batch tiles
+  bool seg;          // four starting points in k
 };
-static HeadPlan head_plan(int B, int V) {
+static HeadPlan head_plan(int B, int D, int V, int64_t ldw) {
   HeadPlan p;
+  // weight rows a multiple of 4096 bytes apart: four starting points in k
+  // (each quarter a whole number of ring turns), for up to 64 batch rows
+  p.seg = B <= 64 && ldw % 2048 == 0 && D % (4 * WIDE_RING * WIDE_SK) == 0;
   p.nt = B <= 32 ? 0 : B <= 64 ? 1 : B <= 128 ? 2 : 3;
   p.nby = (B + (32 << p.nt) - 1) / (32 << p.nt);
   if (p.nt == 0) {
     // small workgroups balance best at every V: 120 against 134 us for 128
     // vocab rows at V = 80000, 11 against 15 us at V = 4080
     p.vt = HEAD_VT_MIN;
+    // head_tall where its tiles fill the CUs in one round and k either is
+    // short or starts at 0 everywhere (B = 32, us, tall against wide: 251
+    // tiles D = 256 17 and 22, 3072 141 and 155; 196 tiles D = 1536 65 and
+    // 72; 167 tiles D = 768 35 and 38, 1536 63 and 63; 147 tiles D = 512 21
+    // and 21, 768 34 and 32; 128 tiles D = 512 22 and 18)
+    const int t = vocab_tiles(V, TALL_VT);
+    if (!p.seg && (D <= 256 ? t >= 144
+                            : t <= 256 && (t >= 192 || (t >= 160 && D <= 768) ||
+                                           (t >= 144 && D <= 512))))
+      p.vt = TALL_VT;
   } else if (p.nt < 3) {
     // 128 vocab rows (B = 64: 57 against 62 us at V = 32000) once they fill
     // most of the CUs; below, 64 (18 against 24 us at V = 16000)
@@ -344,12 +452,27 @@ static HeadPlan head_plan(int B, int V) {
 
 int launch_head(const HeadArgs& A0, hipStream_t s) {
   HeadArgs A = A0;
-  const HeadPlan p = head_plan(A.B, A.V);
+  const HeadPlan p = head_plan(A.B, A.D, A.V, A.ldw);
   A.nvt = vocab_tiles(A.V, p.vt);
-  // weight rows a multiple of 4096 bytes apart: four starting points in k
-  // (each quarter a whole number of ring turns)
-  const bool seg = A.ldw % 2048 == 0 && A.D % (4 * WIDE_RING * WIDE_SK) == 0;
+  const bool seg = p.seg;
   using K = void (*)(HeadArgs);
+  if (p.vt == TALL_VT) {
+    const int v = A.B > 16;
+    static const K tall[2] = {head_tall<1, 3>, head_tall<2, 2>};
+    const int kc = min(A.D, v ? tall_chunk<2>() : tall_chunk<1>());
+    // the dynamic-LDS limit raised once per variant to the most any launch takes
+    static std::once_flag once[2];
+    hipError_t err = hipSuccess;
+    std::call_once(once[v], [&] {
+      err = hipFuncSetAttribute((const void*)tall[v], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                TALL_LDS);
+    });
+    if (err != hipSuccess) return (int)err;
+    timed_launch(CX_KERNEL_LMHEAD, tall[v], dim3((unsigned)A.nvt), dim3(TALL_NW * 64),
+                 (uint32_t)(16 * (v + 1) * (kc + 8) * 2), s, A);
+    timed_launch(CX_KERNEL_LMHEAD_MERGE, head_merge, dim3(A.B), dim3(HEAD_WG), 0, s, A);
+    return (int)hipGetLastError();
+  }
   K k;
   switch (p.nt) {
     case 0: k = seg ? head_wide<2, 1, 4, 4> : head_wide<2, 1, 4, 1>; break;
@@ -394,7 +517,7 @@ int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* w
     return cx::api_fail(CX_EINVAL, "null pointer argument");
   if ((((uintptr_t)hidden | (uintptr_t)weight) & 15) || ((ldh | ldw) & 7))
     return cx::api_fail(CX_EINVAL, "hidden and weight rows must be 16-byte aligned");
-  const size_t need = (size_t)B * cx::vocab_tiles(V, cx::head_plan(B, V).vt) * 8;
+  const size_t need = (size_t)B * cx::vocab_tiles(V, cx::head_plan(B, D, V, ldw).vt) * 8;
   if (ws_bytes < need)
     return cx::api_fail(CX_ENOSPACE, "workspace holds %zu bytes, needs %zu", ws_bytes, need);
   cx::HeadArgs A;

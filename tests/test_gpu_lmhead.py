@@ -90,6 +90,32 @@ def test_tile_edges(B, D, V):
     assert len(set(lg[0, same].tolist())) == 1 and ids[0] == same[0]
 
 
+@pytest.mark.parametrize("B,D,V", [
+    (1, 128, 73729), (16, 256, 73728), (17, 384, 81921), (32, 128, 131585),   # tall tiles of 512
+    (32, 2432, 98305)])                                  # and k in two staged chunks
+def test_tall_tiles(B, D, V):
+    """The 512-row tiles of small batches give the logits of the 64-row batch
+    tile's workgroups (the same order of k), and the greedy id of them."""
+    import torch
+    from chenxing_amd._lib import lmhead_argmax_device
+    print(f"[gpu] lm head tall tiles B={B} D={D} V={V}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(B + D + V)
+    w = (torch.randn(V, D, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    h = torch.randn(33, D, generator=g, device="cuda").to(torch.bfloat16)
+    lg = [torch.empty((n, V), dtype=torch.float32, device="cuda") for n in (B, 33)]
+    ids, mx = lmhead_argmax_device(h[:B], w, out_logits=lg[0])
+    lmhead_argmax_device(h, w, out_logits=lg[1])
+    torch.cuda.synchronize()
+    assert torch.equal(lg[0], lg[1][:B])
+    best = lg[0].max(1)
+    assert torch.equal(ids.long(), (lg[0] == best.values[:, None]).int().argmax(1))
+    assert torch.equal(mx, best.values)
+    exact = h[:B].double() @ w[:4096].double().T
+    tol = H.head_tolerance(_host(h[:B]), _host(w[:4096]))
+    assert (np.abs(lg[0][:, :4096].cpu().numpy() - exact.cpu().numpy()) <= tol).all()
+
+
 def test_ties_and_nan():
     print("[gpu] lm head ties and NaN", flush=True)
     rng = np.random.default_rng(9)
