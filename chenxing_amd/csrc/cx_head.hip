@@ -193,8 +193,10 @@ __global__ __launch_bounds__(NW * 64, 1) void head_wide(HeadArgs A) {
   WideStage<MT> ring[WIDE_RING];
 
   // Request the s-th stage in this workgroup's order (clamped to the last
-  // one, so every stage issues the same number of loads and the counted
-  // waits hold to the end).
+  // one, so every turn of the loop issues the same number of loads and its
+  // counted waits hold to its end).  The hidden states come first: a wait
+  // that leaves the later stages' loads outstanding covers them whatever the
+  // compiler does with the weights, whose own uses wait for them.
   auto request = [&](int s, uint16_t* buf, WideStage<MT>& x) {
     int ks = min(s, S - 1) + rot;
     if (NSEG > 1 && ks >= S) ks -= S;
@@ -262,11 +264,14 @@ __global__ __launch_bounds__(NW * 64, 1) void head_wide(HeadArgs A) {
       step(s + 3, s_h3, ring[3], s_h2, ring[2], acc[j]);
     }
   }
-  if (NSEG == 1 && s < S) {                  // S is even
-    step(s, s_h0, ring[0], s_h3, ring[3], acc[0]);
-    step(s + 1, s_h1, ring[1], s_h0, ring[0], acc[0]);
-  }
   wait_vm<0>();                              // the last requests write LDS: end them first
+  if (NSEG == 1 && s < S) {                  // S is even: two stages left, both requested
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    multiply(s_h0, ring[0], acc[0]);
+    multiply(s_h1, ring[1], acc[0]);
+  }
   // the segments' sums, added in the order of k whatever order they came in
   // (acc[j] is segment (phase + j) % NSEG)
   if (NSEG > 1) {
