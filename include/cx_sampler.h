@@ -227,6 +227,11 @@ int cx_spec_verify_host(const float* target, const float* draft, const int32_t* 
  *  workspace  device scratch of cx_lmhead_workspace_bytes(B, V) bytes; any
  *             contents.  The size grows with B and with V: one workspace of
  *             the largest batch and vocabulary serves every smaller call.
+ * Each logit is an fp32 sum over D.  Its order is the same for every batch of
+ * up to 64 rows and for every larger one, but not for both where ldw is a
+ * multiple of 2048 and D of 1024 (four quarter sums, or one sum, in k order):
+ * there a near tie can go to another id from B = 64 to B = 65, or with the
+ * weight rows padded.
  * Device pointers, stream-ordered, no synchronisation, no allocation.
  */
 int cx_lmhead_argmax_bf16(const uint16_t* hidden, int64_t ldh, const uint16_t* weight,

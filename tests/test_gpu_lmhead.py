@@ -116,6 +116,29 @@ def test_tall_tiles(B, D, V):
     assert (np.abs(lg[0][:, :4096].cpu().numpy() - exact.cpu().numpy()) <= tol).all()
 
 
+@pytest.mark.parametrize("pitch", [1024, 1152, 2048])
+def test_logits_and_batch_size(pitch):
+    """A row's logits are the same bit for bit in every batch of up to 64
+    rows, and in every larger one; in both where the weight pitch is not a
+    multiple of 4096 bytes."""
+    import torch
+    from chenxing_amd._lib import lmhead_argmax_device
+    print(f"[gpu] lm head logits and batch size, pitch {pitch}", flush=True)
+    D, V = 1024, 20611
+    g = torch.Generator(device="cuda")
+    g.manual_seed(pitch)
+    w = (torch.randn(V, pitch, generator=g, device="cuda") * 0.05).to(torch.bfloat16)[:, :D]
+    h = torch.randn(300, D, generator=g, device="cuda").to(torch.bfloat16)
+    got = {}
+    for B in (1, 16, 17, 33, 64, 65, 128, 129, 256, 300):
+        got[B] = torch.empty((B, V), dtype=torch.float32, device="cuda")
+        lmhead_argmax_device(h[:B], w, out_logits=got[B])
+    torch.cuda.synchronize()
+    for B, lg in got.items():
+        same = 64 if B <= 64 and pitch == 2048 else 300
+        assert torch.equal(lg, got[same][:B]), (B, same)
+
+
 def test_ties_and_nan():
     print("[gpu] lm head ties and NaN", flush=True)
     rng = np.random.default_rng(9)
