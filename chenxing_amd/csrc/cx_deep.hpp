@@ -46,12 +46,13 @@
 // Each thread reads 32 bytes per pass step (8 fp32 or 16 bf16 values).  On
 // rows that start at whole dwords (SampleArgs::vec_ok) these are two
 // range-checked buffer loads, issued three steps ahead and unpacked only
-// where used, so the loads stay in flight; bf16 rows at odd addresses load
-// value by value.
+// where used, so the loads stay in flight; other rows (bf16 rows at odd
+// addresses, and fp32 rows of a pointer off a dword address) load value by
+// value.
 //
-// The sums that decide run in a fixed order in fp64.  Each term is within 1 ulp
-// (2.5 ulp for the table product), fp64 sums of at most 2^20 terms within
-// 2^20 ulp, and the reference's own cumulative sums within 4e-11 (relative)
+// The sums that decide run in a fixed order in fp64.  Each term is within
+// 1 ulp (2.5 ulp for the table product), fp64 sums of at most 2^20 terms
+// within 2^20 ulp, and the reference's own cumulative sums within 4e-11 (relative)
 // of exact: a decision closer to its threshold than 5e-11 of the total
 // returns false and the row takes the multi-pass path, as do NaN rows, cuts
 // below the bucket span and cut buckets of more elements than the gather

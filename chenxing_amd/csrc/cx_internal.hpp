@@ -81,8 +81,8 @@ struct SampleArgs {
   int32_t* row_status;
   float* out_probs;
   // [B + 1], each written by the fused kernel before the later kernels read
-  // it: [row] of a sliced row, 0; [row] of a single-slice row, its hand-off
-  // mark (ROW_FINISH, ROW_REFINE,
+  // it: [row] of a sliced row, ROW_WHOLE or 0; [row] of a single-slice row,
+  // its hand-off mark (ROW_WHOLE, ROW_FINISH, ROW_REFINE,
   // ROW_PENDING, or 0 if decided, with MARK_DEEP and MARK_TOPK), which,
   // unlike row_status, the finishing kernels leave as it is; [B],
   // finish16_kernel's work-item counter (zeroed)

@@ -176,8 +176,9 @@ def test_slow_path_rows():
 
 
 def test_penalties_long_window_and_unaligned_rows():
-    """Penalty windows with n_keep, duplicates and out-of-range ids; a row
-    stride that breaks 16-byte alignment (scalar path)."""
+    """Penalty windows with n_keep, duplicates and out-of-range ids; rows of
+    an odd length, so most start off 16-byte boundaries (read as vectors at
+    dword addresses; element loads: test_gpu_whole.py)."""
     rng = np.random.default_rng(5)
     B, V, H = 24, 30001, 3000
     x = rng.normal(0, 2, (B, V)).astype(np.float32)

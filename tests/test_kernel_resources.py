@@ -39,7 +39,7 @@ def _asm(src: str, out: str) -> str:
     return open(out).read()
 
 
-@pytest.mark.parametrize("src", ["cx_sample.hip", "cx_slow.hip", "cx_verify.hip"])
+@pytest.mark.parametrize("src", ["cx_sample.hip", "cx_slow.hip", "cx_verify.hip", "cx_head.hip"])
 def test_kernels_have_no_scratch_and_no_calls(src):
     with tempfile.TemporaryDirectory() as tmp:
         s = _asm(src, os.path.join(tmp, "k.s"))
