@@ -1,6 +1,7 @@
 #include <mutex>
-// Runs what a cx_sample_f32 call runs on the GPU, on the host: the fused
-// kernel (sample_kernel, one workgroup per row slice), then slow_kernel (the
+// Runs what a cx_sample_f32 or cx_sample_bf16 call runs on the GPU, on the
+// host: the fused kernel (sample_kernel, one workgroup per row slice), with
+// bf16 finish16_kernel, then slow_kernel (the
 // region finisher, the refinement, the deep-nucleus and exact multi-pass
 // paths), one workgroup at a time, one OS thread per work-item.  The
 // dynamic LDS of each workgroup is an exact-size allocation of the bytes its
@@ -47,6 +48,7 @@ using namespace cx;
 namespace cx {
 template <bool BF16, bool EXACT> void sample_kernel(SampleArgs A);
 void slow_kernel(SampleArgs A);
+void finish16_kernel(SampleArgs A);
 }  // namespace cx
 
 // The launch geometry and LDS layouts of cx_api.hip (slow_layout,
@@ -173,10 +175,10 @@ int main(int argc, char** argv) {
   int32_t ngroups;
   if (fread(&ngroups, 4, 1, in) != 1) return 2;
   for (int g = 0; g < ngroups; ++g) {
-    int32_t hdr[3];
-    if (fread(hdr, 4, 3, in) != 3) return 2;
-    const int B = hdr[0], V = hdr[1], H = hdr[2];
-    float* x = rd<float>(in, (size_t)B * V);
+    int32_t hdr[4];
+    if (fread(hdr, 4, 4, in) != 4) return 2;
+    const int B = hdr[0], V = hdr[1], H = hdr[2], bf16 = hdr[3], esz = bf16 ? 2 : 4;
+    unsigned char* x = rd<unsigned char>(in, (size_t)B * V * esz);
     cx_row_params* prm = rd<cx_row_params>(in, B);
     int32_t* hist = H > 0 ? rd<int32_t>(in, (size_t)B * H) : nullptr;
     int32_t* hl = H > 0 ? rd<int32_t>(in, B) : nullptr;
@@ -199,14 +201,21 @@ int main(int argc, char** argv) {
     A.nsplit = nsplit;
     A.split_len = split_len_of(V, nsplit);
     A.logV = log((double)V);
-    A.vec_ok = vec_flags(x, (int64_t)V * 4, A.split_len);
+    A.bf16 = bf16;
+    A.vec_ok = vec_flags(x, (int64_t)V * esz, A.split_len);
     slow_layout(A, V, H);
     fused_layout(A, H);
     for (unsigned blk = 0; blk < (unsigned)(B * nsplit); ++blk) {
-      if (nsplit > 1) run_workgroup(sample_kernel<false, true>, A, blk, A.lds_bytes);
-      else run_workgroup(sample_kernel<false, false>, A, blk, A.lds_bytes);
+      run_workgroup(bf16 ? (nsplit > 1 ? sample_kernel<true, true> : sample_kernel<true, false>)
+                         : (nsplit > 1 ? sample_kernel<false, true> : sample_kernel<false, false>),
+                    A, blk, A.lds_bytes);
     }
     const size_t slow_lds = (size_t)std::max(A.slow_lds_bytes, FIN_CAP * 32);
+    if (bf16) {
+      for (unsigned item = 0; item < (unsigned)B; ++item)
+        run_workgroup(finish16_kernel, A, item, (size_t)FIN_CAP * 32);
+      A.pending_only = 1;
+    }
     for (unsigned row = 0; row < (unsigned)B; ++row) run_workgroup(slow_kernel, A, row, slow_lds);
     fwrite(ids, 4, B, out);
     fwrite(st, 4, B, out);

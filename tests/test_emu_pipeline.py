@@ -23,6 +23,7 @@ import pytest
 
 import cases
 from chenxing_amd.params import RowParams, pack_rows
+from chenxing_amd.workloads import bf16_to_f32, f32_to_bf16_rne
 from oracle import sampler_ref as R
 from parity import is_margin
 
@@ -89,8 +90,9 @@ def _params(c) -> RowParams:
                      repetition_penalty=p["repetition_penalty"], n_keep=p["n_keep"])
 
 
-def run_pipeline(groups_in, tmp, env=None):
-    """groups_in: list of case lists (one V each).  Returns [(ids, status)]."""
+def run_pipeline(groups_in, tmp, env=None, bf16=False):
+    """groups_in: list of case lists (one V each); with bf16 their logits,
+    which bf16 holds, go in as bf16.  Returns [(ids, status)]."""
     exe = _build(tmp)
     fin, fout = os.path.join(tmp, "in.bin"), os.path.join(tmp, "out.bin")
     with open(fin, "wb") as f:
@@ -99,8 +101,8 @@ def run_pipeline(groups_in, tmp, env=None):
             B, V = len(cs), cs[0].logits.size
             x = np.stack([c.logits for c in cs]).astype(np.float32)
             H = max(len(c.hist) for c in cs)
-            f.write(struct.pack("iii", B, V, H))
-            f.write(np.ascontiguousarray(x).tobytes())
+            f.write(struct.pack("iiii", B, V, H, int(bf16)))
+            f.write(np.ascontiguousarray(f32_to_bf16_rne(x) if bf16 else x).tobytes())
             f.write(pack_rows([_params(c) for c in cs]).tobytes())
             if H > 0:
                 hist = np.full((B, H), -1, np.int32)
@@ -274,3 +276,35 @@ def test_whole_rows_emulated(V, nsplit):
         assert int(st[b]) & 0xFF == res.status, (c.name, int(st[b]), res.status)
         assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
         assert int(st[b]) >> 8 == (0 if c.params["typical_p"] == 1.0 else 0x5), (c.name, st[b])
+
+
+@pytest.mark.parametrize("V", [33001, 2001, 2006])
+def test_bf16_rows_emulated(V):
+    """bf16 rows at odd addresses (every load a single value), sliced and in
+    one slice, and at dword addresses: unfiltered, typical-p, top-p, a
+    top-k row with a penalty window, masked and NaN rows."""
+    rng = np.random.default_rng(V)
+    base = dict(temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, typical_p=1.0,
+                repetition_penalty=1.0, n_keep=0)
+    rows = []
+    for i, (kw, hist) in enumerate([
+            (dict(), []), (dict(typical_p=0.9), []), (dict(top_p=0.9), []),
+            (dict(top_k=40, top_p=0.9, repetition_penalty=1.2),
+             [int(t) for t in rng.integers(0, V, 50)]),
+            (dict(temperature=0.0), []), (dict(), [])]):
+        x = rng.normal(0.0, 2.0, V).astype(np.float32)
+        if i in (0, 1):
+            x[rng.choice(V, V // 3, replace=False)] = -np.inf
+        if i == 5:
+            x[V - 2] = np.nan
+        rows.append(cases.SamplerCase(f"bf16_{i}", bf16_to_f32(f32_to_bf16_rne(x)),
+                                      dict(base, **kw, seed=int(rng.integers(0, 2**31))), hist))
+    with tempfile.TemporaryDirectory() as tmp:
+        (ids, st), = run_pipeline([rows], tmp, bf16=True)
+    for b, c in enumerate(rows):
+        u = np.random.default_rng(c.params["seed"]).random()
+        res = R.sample_row(c.logits, _params(c), c.hist, u, tie="spread")
+        assert int(st[b]) & 0xFF == res.status, (c.name, int(st[b]), res.status)
+        if res.status != R.STATUS_ERROR:
+            assert int(ids[b]) == res.token or is_margin(res), (c.name, int(ids[b]), res.token)
+    assert int(st[0]) >> 8 == 0                            # drawn from the chunk sums
