@@ -123,12 +123,15 @@ __device__ __forceinline__ void head_keys(const HeadArgs& A, const f32x4 (&acc)[
 //    time.  The workgroups therefore start at different quarters of k and
 //    wrap around.  Each quarter has its own accumulators and the four sums
 //    are added in one fixed order, so a weight row gives the same logit
-//    wherever it lies (equal rows still tie).  Measured at V = 128256,
+//    wherever it lies (equal rows still tie); batches of more than 64 rows,
+//    and other pitches, add one sum in k order.  Measured at V = 128256,
 //    D = 4096: B = 32 213 -> 189 us, B = 64 228 -> 195 us (with rows padded
 //    by 128 bytes: 184 and 195 us); two starts instead of four give nothing,
 //    and for larger batches four sets of accumulators do not fit.
-//  * Measured, B = 256, V = 128256, D = 4096: 291 us, 925 TFLOP/s (1416 us with
-//    32 batch rows per pass over the weights); B = 128 241 us (was 704 us);
+//  * Measured (a call, without a profiler), B = 256, V = 128256, D = 4096: 292
+//    to 297 us, 905 to 921 TFLOP/s (1416 us with 32 batch rows per pass over
+//    the weights); 24 dispatches back to back under the profiler 282 to 395
+//    us, the middle ones longest.  B = 128 241 us (was 704 us);
 //    B = 16, V = 32000 50 us (131 us with 512 vocab rows a workgroup, which
 //    left 193 of the 256 CUs without one).
 constexpr int WIDE_SK = 64;                  // k per stage

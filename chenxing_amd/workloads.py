@@ -14,8 +14,8 @@ deviation s.  Sizes:
   spec_verify     B=32, gamma=8, V=128256: target N(0,2) [B, 9, V], draft =
                   target[:, :8] + N(0, 0.5); draft ids drawn from the draft
                   softmax; T 1.0 or greedy
-  typical         the nucleus logits, T 1.0, typical-p 0.95 (the exact
-                  multi-pass path)
+  typical         the nucleus logits, T 1.0, typical-p 0.95 (chunk sums, then
+                  the deep-nucleus passes in the typical order)
   hetero_bf16     B=1024, V=256000, bf16 of N(0,2) + 10 on 3 ids/row; per-row
                   T ~ U[0.3, 1.5], top-k in {0, 20, 100, 1000},
                   top-p ~ U[0.5, 1.0], 25% of rows greedy

@@ -12,6 +12,7 @@ barrier of theirs checked to be the same one for all work-items.  CPU
 only."""
 from __future__ import annotations
 
+import functools
 import os
 import re
 import shutil
@@ -54,6 +55,13 @@ def _build(tmp: str) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
     return exe
+
+
+@functools.lru_cache(maxsize=1)
+def _exe():
+    """The emulation, built once per run (the directory goes with the run)."""
+    tmp = tempfile.TemporaryDirectory()
+    return _build(tmp.name), tmp
 
 
 def _groups():
@@ -104,7 +112,7 @@ def _run(groups, mode: int = 0, env=None):
     the typical rows' entropy shifts, NaN: the row's own])."""
     us = []
     with tempfile.TemporaryDirectory() as tmp:
-        exe = _build(tmp)
+        exe, _ = _exe()
         fin, fout = os.path.join(tmp, "in.bin"), os.path.join(tmp, "out.bin")
         with open(fin, "wb") as f:
             f.write(struct.pack("i", len(groups)))

@@ -11,6 +11,7 @@ the run; the ids and outcomes must equal the oracle's (margin cases
 counted).  CPU only."""
 from __future__ import annotations
 
+import functools
 import os
 import re
 import shutil
@@ -83,6 +84,13 @@ def _build(tmp: str) -> str:
     return exe
 
 
+@functools.lru_cache(maxsize=1)
+def _exe():
+    """The emulation, built once per run (the directory goes with the run)."""
+    tmp = tempfile.TemporaryDirectory()
+    return _build(tmp.name), tmp
+
+
 def _params(c) -> RowParams:
     p = c.params
     return RowParams(temperature=p["temperature"], top_k=p["top_k"], top_p=p["top_p"],
@@ -93,7 +101,7 @@ def _params(c) -> RowParams:
 def run_pipeline(groups_in, tmp, env=None, bf16=False):
     """groups_in: list of case lists (one V each); with bf16 their logits,
     which bf16 holds, go in as bf16.  Returns [(ids, status)]."""
-    exe = _build(tmp)
+    exe, _ = _exe()
     fin, fout = os.path.join(tmp, "in.bin"), os.path.join(tmp, "out.bin")
     with open(fin, "wb") as f:
         f.write(struct.pack("i", len(groups_in)))
