@@ -270,7 +270,7 @@ __device__ inline bool deep_eligible(const SampleArgs& A, int row, const cx_row_
 // Before, the row was streamed for a region it then outgrew and summed,
 // bucketed and drawn by one workgroup: 64 rows of 128256 fp32, no filter,
 // 108 us a call, now 24.6; typical-p 0.95 on the multi-pass path, 1230 us, now
-// 116 (deep_row below).
+// 117 (deep_row below).
 struct WholePart {
   double s;          // sum of exp((x - m) / T) over the chunk (NaN: a NaN or +inf element)
   double sd;         // sum of exp((x - m) / T) (x - m) / T
